@@ -256,12 +256,12 @@ constexpr int kMaxOpBatch = 512;  // the reference's largest batched tile (Mp <=
 
 void launch_linear(xe_ctx *ctx, const xe_weight *w, const void *x, int x_dtype, int batch,
                    float *y, hipStream_t s) {
+  const GemvLaunch L = gemv_args(w, x, x_dtype, batch, y);
   if (!gemm_preferred(w->m, w->k, batch)) {
-    launch_gemv(gemv_args(w, x, x_dtype, batch, y), s);
+    launch_gemv(L, s);
   } else {
-    // the prologue (norm, or bf16 x to fp32) writes batch x k floats
-    ctx->ensure_gemm(w->norm != XE_NORM_NONE || x_dtype == XE_BF16 ? static_cast<size_t>(batch) * w->k : 0);
-    launch_gemm_op(gemv_args(w, x, x_dtype, batch, y), ctx->gemm_xn, ctx->gemm_ws, ctx->gemm_cnt, s);
+    ctx->ensure_gemm(gemm_op_xn_floats(L));
+    launch_gemm_op(L, ctx->gemm_xn, ctx->gemm_ws, ctx->gemm_cnt, s);
   }
   ctx->dispatches++;
 }
@@ -1072,8 +1072,12 @@ int xe_probe_gemv(xe_ctx *ctx, const xe_weight *const *ws, int n_weights, const 
       XE_REQUIRE(ws[i]->m == ws[0]->m && ws[i]->k == ws[0]->k, "probe weights differ in shape");
     }
     DeviceGuard dg(ctx->dev->ordinal);
-    if (gemm_preferred(ws[0]->m, ws[0]->k, batch))
-      ctx->ensure_gemm(static_cast<size_t>(batch) * ws[0]->k);  // no allocation under capture
+    if (gemm_preferred(ws[0]->m, ws[0]->k, batch)) {  // no allocation under capture
+      size_t xn = 0;
+      for (int i = 0; i < n_weights; i++)
+        xn = std::max(xn, gemm_op_xn_floats(gemv_args(ws[i], x_dev, x_dtype, batch, y_dev)));
+      ctx->ensure_gemm(xn);
+    }
     const double us = time_captured(ctx, reps, flags, [&]() {
       for (int i = 0; i < n_weights; i++)
         launch_linear(ctx, ws[i], x_dev, x_dtype, batch, y_dev, ctx->dev->stream);

@@ -31,6 +31,7 @@
 // runs as its own kernel, one workgroup per stream row, writing the
 // normalised activations that the GEMM reads.
 #include "gemv_dev.h"
+#include "wide.h"
 
 namespace xe {
 namespace {
@@ -1460,9 +1461,41 @@ void launch_gemm(const gdev::GemvParams &p, int wdtype, float *ws, unsigned *cnt
 size_t gemm_op_ws_floats() { return kGemmWsFloats; }
 size_t gemm_op_cnt_words() { return kGemmMaxTiles; }
 
+namespace {
+bool op_wide(const GemvLaunch &L) {
+  return L.act == ACT_NONE && !L.sub && !L.res_out && L.out_scale == 1.0f &&
+         wide_preferred(L.m, L.k, L.batch) && wide_takes(L.m, L.k, L.batch, L.wdtype, L.x, L.ldx);
+}
+}  // namespace
+
+size_t gemm_op_xn_floats(const GemvLaunch &L) {
+  if (op_wide(L)) return wide_rows_floats(L.wdtype, L.batch, L.k);
+  return gemm_needs_prologue(gdev::to_params(L)) ? static_cast<size_t>(L.batch) * L.k : 0;
+}
+
 void launch_gemm_op(const GemvLaunch &L, float *xn, float *ws, unsigned *cnt, hipStream_t s) {
   XE_REQUIRE(L.x_dtype == XE_F32 || L.x_dtype == XE_BF16, "gemm: fp32 or bf16 activations");
   gdev::GemvParams p = gdev::to_params(L);
+  if (op_wide(L)) {
+    XE_REQUIRE(xn, "gemm: no buffer for the row planes");
+    WideGemm g;
+    g.wdtype = L.wdtype;
+    g.w = L.w;
+    g.scale = L.scale;
+    g.exps = L.exps;
+    g.bias = L.bias;
+    g.m = L.m;
+    g.k = L.k;
+    g.n = L.batch;
+    g.rows = wide_rows_in(xn, L.batch);
+    g.y = L.y;
+    g.ldy = L.ldy;
+    g.ws = ws;
+    g.ws_floats = kGemmWsFloats;
+    launch_wide_rows(p, L.wdtype, g.rows, s);
+    launch_wide_gemm(g, s);
+    return;
+  }
   if (gemm_needs_prologue(p)) {  // bf16 x: the prologue writes it as fp32
     XE_REQUIRE(xn, "gemm: prologue without a row buffer");
     launch_gemm_prologue(p, xn, s);

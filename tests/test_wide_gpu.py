@@ -1,14 +1,20 @@
-"""Many rows at once: the plane GEMM of large op-layer batches.
+"""Many rows at once: the plane GEMM of large op-layer batches, and prompts fed
+in passes over all their tokens.
 
-Compared with a float64 product of the same stored weights (bar: rel-L2 1e-6,
-an fp32 sum's rounding at these K: about 2^-24 sqrt(K) / 4), at sizes that
-leave remainders in every tile: rows modulo 64 and 128, weight rows modulo 64
-and 256, K modulo 64.
+The GEMM is compared with a float64 product of the same stored weights
+(bar: rel-L2 1e-6, an fp32 sum's rounding at these K: about 2^-24 sqrt(K) / 4),
+at sizes that leave remainders in every tile: rows modulo 64 and 128, weight
+rows modulo 64 and 256, K modulo 64.  Prompts are compared with the oracle's
+token-by-token logits (the bars of parity_util), at row counts either side of
+the plane kernels' first one, over several key tiles and over more rows than
+one pass takes.
 """
 import numpy as np
 import pytest
 
 import oracle_lib as O
+from parity_util import compare_logits
+from test_decoder_gpu import build, prompts, tiny
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +61,30 @@ def test_wide_linear(gpu, xe, wd, m, k, b, norm):
     # row by row: a row's exponent, padding or order mixed up shows here
     rows = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
     assert rows.max() <= 2e-6, "row %d rel-L2 %g" % (rows.argmax(), rows.max())
+
+
+def prompt_cfg(xe, family, wd):
+    wdtype = {"i8": xe.XE_I8, "bf16": xe.XE_BF16, "bfp16": xe.XE_BFP16}[wd]
+    cfg = tiny(xe, {"opt": xe.XE_OPT, "whisper": xe.XE_WHISPER}.get(family, xe.XE_GEMMA3), wdtype)
+    if family == "gemma_hd128":
+        cfg = cfg.replace(n_heads=4, n_kv_heads=2, head_dim=128)
+    return cfg
+
+
+@pytest.mark.parametrize("family,wd,batch,n", [
+    ("gemma", "i8", 1, 4), ("gemma", "i8", 1, 65), ("gemma", "i8", 1, 66), ("gemma", "bf16", 3, 50),
+    ("gemma", "i8", 2, 330), ("gemma_hd128", "i8", 2, 70), ("gemma", "bfp16", 22, 4),
+    ("opt", "i8", 1, 70), ("opt", "bfp16", 5, 40), ("opt", "i8", 20, 111),
+    ("whisper", "i8", 1, 5), ("whisper", "i8", 7, 29), ("whisper", "bf16", 3, 80)])
+def test_prompt_passes_logits(gpu, xe, family, wd, batch, n):
+    cfg = prompt_cfg(xe, family, wd)
+    print("[case] prompt %s %s batch %d, %d tokens" % (family, wd, batch, n), flush=True)
+    dec, om = build(xe, gpu, cfg, seed=31, batch=batch)
+    pr = prompts(cfg, batch, n, seed=n)
+    dec.feed(pr[:, :-1])
+    got, _ = dec.step(pr[:, -1], np.full(batch, n - 1, np.int32))
+    for p in range(n):
+        want = om.step(pr[:, p], np.full(batch, p, np.int32))
+    compare_logits(got, want, "prompt-%s-%s-b%d-n%d" % (family, wd, batch, n))
+    dec.close()
+    om.close()

@@ -24,8 +24,10 @@
 #include <memory>
 
 #include "ll_dev.h"
+#include "prefill.h"
 #include "quant.h"
 #include "step_dev.h"
+#include "wide.h"
 
 namespace xe {
 namespace {
@@ -387,6 +389,10 @@ struct xe_decoder {
     hipGraphExec_t graph = nullptr;
   };
   std::map<int, Plan> plans;
+  std::map<int, Plan> tails;  // final norm, lm-head and argmax of a prompt's last rows (launched eagerly)
+  // workspace of prompt passes (PromptWs): one allocation, grown on demand
+  char *prompt_ws = nullptr;
+  size_t prompt_ws_bytes = 0;
   // low-latency executor (ll_dev.h): one plan per batch size
   struct LLPlan {
     bool ok = false;
@@ -659,6 +665,7 @@ void drop_plans(xe_decoder *d) {
     if (kv.second.graph) (void)hipGraphExecDestroy(kv.second.graph);
   }
   d->plans.clear();
+  d->tails.clear();
   for (auto &kv : d->ll_plans) {
     if (kv.second.dev_a) (void)hipFree(kv.second.dev_a);
     if (kv.second.dev_f) (void)hipFree(kv.second.dev_f);
@@ -672,6 +679,7 @@ void free_decoder(xe_decoder *d) {
   for (void *p : d->ll_fc2t)
     if (p) (void)hipFree(p);
   if (d->ll_forced) (void)hipFree(d->ll_forced);
+  if (d->prompt_ws) (void)hipFree(d->prompt_ws);
   if (d->step_status) (void)hipFree(d->step_status);
   d->emb.release();
   for (auto &l : d->L) {
@@ -900,6 +908,78 @@ struct PlanBuilder {
   }
 };
 
+// Embedding of n rows: tokens and positions on the device, into x [n, d_model].
+sdev::Phase embed_phase(xe_decoder *d, int n, const int32_t *tokens, const int32_t *pos, float *x) {
+  const auto &c = d->c;
+  sdev::Phase ph{};
+  ph.kind = sdev::PH_EMBED;
+  Spec sp;
+  sdev::EmbedParams &e = ph.u.emb;
+  e.emb = d->emb.w;
+  e.emb_scale = d->emb.scale;
+  e.emb_exps = d->emb.exps;
+  e.wdtype = c.wdtype;
+  e.pos_emb = d->pos_emb;
+  e.pos_off = c.family == XE_OPT ? 2 : 0;
+  e.pos_rows = tensor_spec(c, XE_T_POS_EMB, -1, sp) ? sp.rows : 1;
+  e.mul = sqrtf(static_cast<float>(c.d_model));
+  e.use_mul = c.family == XE_GEMMA3 ? 1 : 0;
+  e.tokens = tokens;
+  e.pos = pos;
+  e.vocab = c.vocab;
+  e.d = c.d_model;
+  e.batch = n;
+  e.x = x;
+  ph.nblocks = n * ((c.d_model + 255) / 256);
+  return ph;
+}
+
+// The end of a step's plan: final norm (after the residual update x + sub,
+// post-normed with post_w when given) + tied lm-head, then the argmax.
+void build_tail(xe_decoder *d, int B, PlanBuilder &pb, const float *x, const float *sub, const float *post_w) {
+  const auto &c = d->c;
+  const bool gem = c.family == XE_GEMMA3, opt = c.family == XE_OPT;
+  {
+    GemvCall g;
+    g.m = &d->emb;
+    g.x = x;
+    g.ldx = c.d_model;
+    g.sub = sub;
+    g.post_w = post_w;
+    g.norm = gem ? XE_NORM_RMS1P : XE_NORM_LN;
+    g.gamma = d->lnf_w;
+    g.beta = gem ? nullptr : d->lnf_b;
+    g.eps = c.eps;
+    g.y = d->logits;
+    g.ldy = c.vocab;
+    pb.gemv(g, B, "gemv_lmhead");
+  }
+  // ---- greedy argmax -> next token, pos + 1 ----
+  {
+    sdev::Phase ph{};
+    sdev::ArgmaxParams &ap = ph.u.arg;
+    ap.logits = d->logits;
+    ap.vocab = c.vocab;
+    ap.batch = B;
+    ap.last_max = opt ? 1 : 0;
+    ap.part_v = d->arg_v;
+    ap.part_i = d->arg_i;
+    ap.next = d->next;
+    ap.tokens = d->tokens;
+    ap.pos = d->pos;
+    ap.hist = d->hist;
+    ap.hist_stride = c.max_ctx + 1;
+    ap.stop = d->stop_dev;
+    ap.done = d->stop_dev + 1;
+    ph.kind = sdev::PH_ARGMAX_PART;
+    ph.nblocks = B * sdev::kArgBlocks;
+    pb.push(ph, "argmax", 4.0 * B * c.vocab);
+    ph.kind = sdev::PH_ARGMAX_FINAL;
+    ph.nblocks = B;
+    pb.push(ph, "argmax_final", 8.0 * B * sdev::kArgBlocks);
+  }
+}
+
 // The phase list of one decode step for streams [0, B) (tokens/pos on device).
 void build_plan(xe_decoder *d, int B, xe_decoder::Plan &plan) {
   const auto &c = d->c;
@@ -912,30 +992,8 @@ void build_plan(xe_decoder *d, int B, xe_decoder::Plan &plan) {
   // the split attention kernel merges in place (arrival counters)
   unsigned *attn_cnt = d->attn_cnt;
 
-  // embedding
-  {
-    sdev::Phase ph{};
-    ph.kind = sdev::PH_EMBED;
-    Spec sp;
-    sdev::EmbedParams &e = ph.u.emb;
-    e.emb = d->emb.w;
-    e.emb_scale = d->emb.scale;
-    e.emb_exps = d->emb.exps;
-    e.wdtype = c.wdtype;
-    e.pos_emb = d->pos_emb;
-    e.pos_off = opt ? 2 : 0;
-    e.pos_rows = tensor_spec(c, XE_T_POS_EMB, -1, sp) ? sp.rows : 1;
-    e.mul = sqrtf(static_cast<float>(D));
-    e.use_mul = gem ? 1 : 0;
-    e.tokens = d->tokens;
-    e.pos = d->pos;
-    e.vocab = c.vocab;
-    e.d = D;
-    e.batch = B;
-    e.x = d->xa;
-    ph.nblocks = B * ((D + 255) / 256);
-    pb.push(ph, "embed", static_cast<double>(B) * D * (wbytes(c.wdtype, 1) + 4 + (d->pos_emb ? 4 : 0)));
-  }
+  pb.push(embed_phase(d, B, d->tokens, d->pos, d->xa), "embed",
+          static_cast<double>(B) * D * (wbytes(c.wdtype, 1) + 4 + (d->pos_emb ? 4 : 0)));
   float *xcur = d->xa, *xalt = d->xb;
   const float *pend = nullptr, *pend_post = nullptr;
   auto take_pending = [&](GemvCall &g) {
@@ -1091,44 +1149,7 @@ void build_plan(xe_decoder *d, int B, xe_decoder::Plan &plan) {
       pend_post = gem ? l.post_ffn : nullptr;
     }
   }
-  // ---- final norm + tied lm-head ----
-  {
-    GemvCall g;
-    g.m = &d->emb;
-    take_pending(g);
-    g.res_out = nullptr;  // the residual is not needed after the head
-    g.norm = norm;
-    g.gamma = d->lnf_w;
-    g.beta = gem ? nullptr : d->lnf_b;
-    g.eps = c.eps;
-    g.y = d->logits;
-    g.ldy = c.vocab;
-    pb.gemv(g, B, "gemv_lmhead");
-  }
-  // ---- greedy argmax -> next token, pos + 1 ----
-  {
-    sdev::Phase ph{};
-    sdev::ArgmaxParams &ap = ph.u.arg;
-    ap.logits = d->logits;
-    ap.vocab = c.vocab;
-    ap.batch = B;
-    ap.last_max = opt ? 1 : 0;
-    ap.part_v = d->arg_v;
-    ap.part_i = d->arg_i;
-    ap.next = d->next;
-    ap.tokens = d->tokens;
-    ap.pos = d->pos;
-    ap.hist = d->hist;
-    ap.hist_stride = c.max_ctx + 1;
-    ap.stop = d->stop_dev;
-    ap.done = d->stop_dev + 1;
-    ph.kind = sdev::PH_ARGMAX_PART;
-    ph.nblocks = B * sdev::kArgBlocks;
-    pb.push(ph, "argmax", 4.0 * B * c.vocab);
-    ph.kind = sdev::PH_ARGMAX_FINAL;
-    ph.nblocks = B;
-    pb.push(ph, "argmax_final", 8.0 * B * sdev::kArgBlocks);
-  }
+  build_tail(d, B, pb, xcur, pend, pend_post);
 }
 
 xe_decoder::Plan &plan_for(xe_decoder *d, int B) {
@@ -1769,6 +1790,284 @@ void run_gemv_now(const GemvCall &g, int batch, hipStream_t s) {
   for (const auto &ph : tmp.phases) launch_phase(ph, s);
 }
 
+// ---------------------------------------------------------------------------
+// prompts: every token of a prompt in one pass
+// ---------------------------------------------------------------------------
+// The rows of a pass: at most kPromptRows tokens over all streams (a longer
+// prompt runs in chunks of tokens); the weights are read once a pass instead
+// of once a token.
+constexpr int kPromptRows = 2048;
+constexpr int kPromptWideRows = 65;
+
+// Device workspace of a prompt pass of up to `rows` rows, one allocation.
+struct PromptWs {
+  float *x[2], *sub, *qkv, *att, *ffn, *qx, *rows, *part;
+  unsigned *cnt;
+  int32_t *tok, *pos;
+  bool wide;  // every linear suits the plane kernels (wide.hip)
+};
+
+PromptWs prompt_ws(xe_decoder *d, int rows) {
+  const auto &c = d->c;
+  const size_t D = c.d_model, hq = static_cast<size_t>(c.n_heads) * c.head_dim, R = rows;
+  const int kmax = static_cast<int>(std::max(std::max(D, hq), static_cast<size_t>(c.ffn)));
+  // row planes (wide.hip), or the normalised rows of gemm.hip
+  const size_t plane = std::max(wide_rows_floats(c.wdtype, rows, kmax), R * kmax);
+  PromptWs w{};
+  size_t off = 0;
+  auto take = [&](size_t floats) {
+    const size_t at = off;
+    off += (floats * 4 + 255) / 256 * 256;
+    return at;
+  };
+  const size_t o_x0 = take(R * D), o_x1 = take(R * D), o_sub = take(R * D), o_qkv = take(R * d->nqkv());
+  const size_t o_att = take(R * std::max(hq, D)), o_ffn = take(R * std::max(static_cast<size_t>(c.ffn), d->nqkv())), o_qx = take(R * D), o_rows = take(plane);
+  const size_t o_part = take(gemm_ws_floats()), o_cnt = take(gemm_cnt_words()), o_tok = take(R), o_pos = take(R);
+  if (off > d->prompt_ws_bytes) {
+    XE_HIP(hipStreamSynchronize(d->s));
+    if (d->prompt_ws) XE_HIP(hipFree(d->prompt_ws));
+    d->prompt_ws = nullptr;
+    d->prompt_ws_bytes = 0;
+    XE_HIP(hipMalloc(reinterpret_cast<void **>(&d->prompt_ws), off));
+    d->prompt_ws_bytes = off;
+  }
+  char *b = d->prompt_ws;
+  auto at = [&](size_t o) { return reinterpret_cast<float *>(b + o); };
+  w.x[0] = at(o_x0), w.x[1] = at(o_x1), w.sub = at(o_sub), w.qkv = at(o_qkv), w.att = at(o_att), w.ffn = at(o_ffn);
+  w.qx = at(o_qx), w.rows = at(o_rows), w.part = at(o_part), w.cnt = reinterpret_cast<unsigned *>(at(o_cnt));
+  w.wide = wide_takes(std::max(std::max(static_cast<int>(d->nqkv()), c.d_model), 2 * c.ffn), kmax, rows, c.wdtype, b, 0);
+  w.tok = reinterpret_cast<int32_t *>(at(o_tok)), w.pos = reinterpret_cast<int32_t *>(at(o_pos));
+  return w;
+}
+
+// A sublayer output on its way into the residual: a buffer, or the K splits
+// of its GEMM with what the GEMM's epilogue would have applied.
+struct Pending {
+  const float *sub = nullptr, *post_w = nullptr;
+  const float *part = nullptr, *scale = nullptr, *bias = nullptr;
+  int ks = 0;
+};
+
+// One linear of a prompt pass over n rows, now.  out: where the result may be
+// left as split partials for the next prologue (null: always in g.y).
+void prompt_linear(xe_decoder *d, const PromptWs &w, GemvCall g, int n, const Pending *in, Pending *out) {
+  const Mat &m = *g.m;
+  // from kPromptWideRows rows the plane kernels; below, the decode step's own
+  if (n < kPromptWideRows || !w.wide) {
+    if (in) {
+      g.sub = in->sub;
+      g.post_w = in->post_w;
+    }
+    xe_decoder::Plan tmp;
+    PlanBuilder pb{tmp, w.rows, w.part, w.cnt};
+    pb.gemv(g, n, "prompt");
+    for (const auto &ph : tmp.phases) launch_phase(ph, d->s);
+    if (out) out->sub = g.y;
+    return;
+  }
+  gdev::GemvParams p{};
+  p.x = g.x;
+  p.ldx = g.ldx;
+  p.batch = n;
+  p.k = m.cols;
+  p.norm = g.norm;
+  p.gamma = g.gamma;
+  p.beta = g.beta;
+  p.eps = g.eps;
+  p.res_out = g.res_out;
+  p.sub_out_scale = 1.0f;
+  if (in) {
+    p.sub = in->sub;
+    p.post_w = in->post_w;
+    p.sub_part = in->part;
+    p.sub_ks = in->ks;
+    p.sub_scale = in->scale;
+    p.sub_bias = in->bias;
+  }
+  WideGemm q;
+  q.wdtype = m.wdtype;
+  q.w = m.w;
+  q.scale = m.scale;
+  q.exps = m.exps;
+  q.bias = g.bias;
+  q.m = m.rows;
+  q.k = m.cols;
+  q.n = n;
+  q.rows = wide_rows_in(w.rows, n);
+  q.act = g.act;
+  q.y = g.y;
+  q.ldy = g.ldy;
+  q.ws = w.part;
+  q.ws_floats = gemm_ws_floats();
+  launch_wide_rows(p, m.wdtype, q.rows, d->s);
+  const int ks = out ? wide_splits(q.m, q.k, n, q.wdtype, q.ws_floats) : 1;
+  if (ks > 1) {
+    q.part = w.part;
+    out->part = w.part;
+    out->ks = ks;
+    out->scale = m.wdtype == XE_I8 ? m.scale : nullptr;
+    out->bias = g.bias;
+  } else if (out) {
+    out->sub = g.y;
+  }
+  launch_wide_gemm(q, d->s);
+}
+
+// Tokens [t0, t0 + t_n) of every stream through the layers (rows already
+// named by w.tok / w.pos).  The last layer ends once every K / V row is
+// appended; in the prompt's last chunk (last) it goes on with the rows of the
+// last tokens, which end in d->xa with their last sublayer output in d->sub.
+void prompt_chunk(xe_decoder *d, const PromptWs &w, int B, int t0, int t_n, bool last) {
+  const auto &c = d->c;
+  const int D = c.d_model, F = c.ffn, hd = c.head_dim;
+  const int hq = c.n_heads * hd, hk = c.n_kv_heads * hd, nq = static_cast<int>(d->nqkv());
+  const bool gem = c.family == XE_GEMMA3, wh = c.family == XE_WHISPER, opt = c.family == XE_OPT;
+  const int norm = gem ? XE_NORM_RMS1P : XE_NORM_LN;
+  int n = B * t_n;
+  launch_phase(embed_phase(d, n, w.tok, w.pos, w.x[0]), d->s);
+  float *x = w.x[0], *alt = w.x[1];
+  Pending pend;
+  bool have = false;
+  auto linear = [&](const Mat &m, const float *bias, float *y, int ldy, const float *gamma, const float *beta, int act,
+                    const float *src, int lds, bool defer) {
+    GemvCall g;
+    g.m = &m;
+    g.bias = bias;
+    g.y = y;
+    g.ldy = ldy;
+    g.act = act;
+    g.eps = c.eps;
+    g.x = src ? src : x;
+    g.ldx = src ? lds : D;
+    if (!src) {
+      g.norm = norm;
+      g.gamma = gamma;
+      g.beta = beta;
+      if (have) g.res_out = alt;
+    }
+    const Pending in = pend;
+    const bool take = !src && have;
+    Pending out;
+    prompt_linear(d, w, g, n, take ? &in : nullptr, defer ? &out : nullptr);
+    if (take) {
+      std::swap(x, alt);
+      have = false;
+    }
+    if (defer) {
+      pend = out;
+      have = true;
+    }
+  };
+  for (int li = 0; li < c.n_layers; li++) {
+    Layer &l = d->L[li];
+    linear(l.qkv, gem ? nullptr : l.qkv_b, w.qkv, nq, l.ln1_w, gem ? nullptr : l.ln1_b, ACT_NONE, nullptr, 0, false);
+    PromptAttn a;
+    a.qkv = w.qkv;
+    a.ldq = nq;
+    a.k_off = hq;
+    a.v_off = hq + hk;
+    a.kc = d->kc + d->kv_layer_elems() * li;
+    a.vc = d->vc + d->kv_layer_elems() * li;
+    a.kv_bstride = static_cast<size_t>(c.n_kv_heads) * c.max_ctx * hd;
+    a.max_ctx = c.max_ctx;
+    a.batch = B;
+    a.t_n = t_n;
+    a.t0 = t0;
+    a.hq = c.n_heads;
+    a.hkv = c.n_kv_heads;
+    a.hd = hd;
+    a.scale = opt ? powf(static_cast<float>(hd), -0.5f) : 1.0f / sqrtf(static_cast<float>(hd));
+    if (gem) {
+      a.q_norm_w = l.qn;
+      a.k_norm_w = l.kn;
+      a.norm_eps = c.eps;
+      a.rope_cos = d->rope_cos;
+      a.rope_sin = d->rope_sin;
+    }
+    a.div_norm = opt ? 1 : 0;
+    a.out = w.att;
+    a.ld_out = hq;
+    launch_prompt_append(a, d->s);
+    const bool end = li == c.n_layers - 1;
+    if (end && !last) return;  // every K / V row of the chunk is in the caches
+    if (end && t_n > 1) {  // from here on the last tokens' rows
+      launch_last_rows(w.qkv, w.ffn, B, t_n, nq, d->s);
+      launch_last_rows(x, alt, B, t_n, D, d->s);
+      std::swap(x, alt);
+      a.qkv = w.ffn;
+      a.t0 = t0 + t_n - 1;
+      a.t_n = 1;
+      n = B;
+    }
+    launch_prompt_attn(a, d->s);
+    linear(l.o, gem ? nullptr : l.o_b, w.sub, D, nullptr, nullptr, ACT_NONE, w.att, hq, true);
+    pend.post_w = gem ? l.post_attn : nullptr;
+    if (wh) {
+      linear(l.xq, l.xq_b, w.qx, D, l.lnx_w, l.lnx_b, ACT_NONE, nullptr, 0, false);
+      PromptAttn xa;
+      xa.qkv = w.qx;
+      xa.ldq = D;
+      xa.kc = l.ck;
+      xa.vc = l.cv;
+      xa.max_ctx = c.n_cross;
+      xa.t_n = n;  // one encoder output for every stream: all rows are queries of one cache
+      xa.hq = xa.hkv = c.n_heads;
+      xa.hd = hd;
+      xa.scale = 1.0f / sqrtf(static_cast<float>(hd));
+      xa.fixed_len = c.n_cross;
+      xa.out = w.att;
+      xa.ld_out = D;
+      launch_prompt_attn(xa, d->s);
+      linear(l.xo, l.xo_b, w.sub, D, nullptr, nullptr, ACT_NONE, w.att, D, true);
+    }
+    linear(l.fc1, gem ? nullptr : l.fc1_b, w.ffn, F, l.ln2_w, gem ? nullptr : l.ln2_b,
+           gem ? ACT_GEGLU_TANH : (opt ? ACT_RELU : ACT_GELU_ERF), nullptr, 0, false);
+    // the last sublayer output stays whole: the lm-head's prologue adds it
+    linear(l.fc2, gem ? nullptr : l.fc2_b, end ? d->sub : w.sub, D, nullptr, nullptr, ACT_NONE, w.ffn, F, !end);
+    pend.post_w = gem ? l.post_ffn : nullptr;
+  }
+  XE_HIP(hipMemcpyAsync(d->xa, x, static_cast<size_t>(B) * D * 4, hipMemcpyDeviceToDevice, d->s));
+}
+
+// Whether feed() runs a prompt in passes instead of token by token.
+bool prompt_in_passes(xe_decoder *d, int batch, int n_prompt) {
+  const auto &c = d->c;
+  if (d->cross_i8k || d->cross_i8v) return false;  // int8 cross rows: the single-query kernels read them
+  return n_prompt >= 3 && batch <= kPromptRows && prompt_attn_takes(c.head_dim, c.n_heads / c.n_kv_heads);
+}
+
+// The prompt in passes over up to kPromptRows rows; h: pinned staging.
+void feed_passes(xe_decoder *d, const int32_t *prompt, int n_prompt, int batch, int32_t *h) {
+  const int tc = std::max(1, std::min(n_prompt, kPromptRows / batch));
+  const PromptWs w = prompt_ws(d, batch * tc);
+  XE_HIP(hipMemsetAsync(w.cnt, 0, gemm_cnt_words() * sizeof(unsigned), d->s));
+  size_t at = 0;
+  for (int t0 = 0; t0 < n_prompt; t0 += tc) {
+    const int t_n = std::min(tc, n_prompt - t0), n = batch * t_n;
+    int32_t *ht = h + at, *hp = ht + n;
+    at += 2 * static_cast<size_t>(n);
+    for (int b = 0; b < batch; b++)
+      for (int t = 0; t < t_n; t++) {
+        ht[b * t_n + t] = prompt[static_cast<size_t>(b) * n_prompt + t0 + t];
+        hp[b * t_n + t] = t0 + t;
+      }
+    XE_HIP(hipMemcpyAsync(w.tok, ht, n * 4, hipMemcpyHostToDevice, d->s));
+    XE_HIP(hipMemcpyAsync(w.pos, hp, n * 4, hipMemcpyHostToDevice, d->s));
+    prompt_chunk(d, w, batch, t0, t_n, t0 + t_n == n_prompt);
+  }
+  int32_t *hp = h + at;
+  for (int b = 0; b < batch; b++) hp[b] = n_prompt - 1;
+  XE_HIP(hipMemcpyAsync(d->pos, hp, batch * 4, hipMemcpyHostToDevice, d->s));
+  auto it = d->tails.find(batch);
+  if (it == d->tails.end()) {
+    it = d->tails.emplace(batch, xe_decoder::Plan{}).first;
+    PlanBuilder pb{it->second, d->gemm_ws ? d->xn : nullptr, d->gemm_ws, d->gemm_cnt, d->gemm_xd, d->gemm_xe, d->c.d_model};
+    build_tail(d, batch, pb, d->xa, d->sub, d->c.family == XE_GEMMA3 ? d->L.back().post_ffn : nullptr);
+  }
+  for (const auto &ph : it->second.phases) launch_phase(ph, d->s);
+  XE_HIP(hipStreamSynchronize(d->s));
+}
+
 // After a run of low-latency launches: a wait that timed out (or a plan the
 // kernel could not run) leaves the status word set; report it and clear it.
 void check_step_status(xe_decoder *d) {
@@ -2334,8 +2633,9 @@ void check_ready(xe_decoder *d, int batch) {
   XE_REQUIRE(d->c.family != XE_WHISPER || d->cross_ready, "Whisper: set_cross first");
 }
 
-// Positions start at 0; the prompt's tokens are fed one step at a time (the
-// argmax kernel leaves the next token and pos + 1 on the device).
+// Positions start at 0; the prompt runs in passes over all its tokens, or (a
+// short one) one step at a time; either way the last token's argmax leaves
+// the next token and pos + 1 on the device.
 void feed(xe_decoder *d, const int32_t *prompt, int n_prompt, int batch) {
   check_ready(d, batch);
   XE_REQUIRE(prompt && n_prompt >= 1, "empty prompt");
@@ -2347,6 +2647,13 @@ void feed(xe_decoder *d, const int32_t *prompt, int n_prompt, int batch) {
   int32_t *h = d->host_tok;
   XE_REQUIRE(static_cast<size_t>(n_prompt + 1) * batch <= static_cast<size_t>(2) * (d->c.max_ctx + 2) * d->max_batch,
              "prompt too long for staging");
+  if (prompt_in_passes(d, batch, n_prompt)) {
+    XE_HIP(hipMemsetAsync(d->stop_dev + 1, 0, batch * 4, d->s));  // no stream has stopped
+    feed_passes(d, prompt, n_prompt, batch, h);
+    for (int b = 0; b < batch; b++) d->hpos[b] = n_prompt;
+    d->live = batch;
+    return;
+  }
   for (int p = 0; p < n_prompt; p++)
     for (int b = 0; b < batch; b++) h[static_cast<size_t>(p) * batch + b] = prompt[static_cast<size_t>(b) * n_prompt + p];
   int32_t *zpos = h + static_cast<size_t>(n_prompt) * batch;

@@ -2142,28 +2142,67 @@ void upload_matrix(xe_decoder *d, const Spec &sp, const Place &p, const float *w
 void precompute_cross(xe_decoder *d) {
   const auto &c = d->c;
   const int D = c.d_model, T = c.n_cross;
-  float *tmp = dalloc<float>(static_cast<size_t>(T) * D, d->s, false);
+  // the projections in fp32, the encoder rows' planes, K-split partials
+  const bool wide = wide_takes(D, D, T, c.wdtype, d->enc, D);
+  const bool quant = d->cross_i8k || d->cross_i8v;
+  const size_t n_tmp = !wide || quant ? (static_cast<size_t>(T) * D + 63) / 64 * 64 : 0;
+  const size_t n_rows = wide ? (wide_rows_floats(c.wdtype, T, D) + 63) / 64 * 64 : 0;
+  float *tmp = dalloc<float>(n_tmp + n_rows, d->s, false);
   struct Free {
     float *p;
     ~Free() { (void)hipFree(p); }
   } fr{tmp};
+  const WideRows rows = wide_rows_in(tmp + n_tmp, T);
+  if (wide) {
+    gdev::GemvParams p{};
+    p.x = d->enc;
+    p.ldx = D;
+    p.batch = T;
+    p.k = D;
+    launch_wide_rows(p, c.wdtype, rows, d->s);
+  }
   for (int li = 0; li < c.n_layers; li++) {
     Layer &l = d->L[li];
     for (int which = 0; which < 2; which++) {
-      GemvCall g;
-      g.m = which == 0 ? &l.xk : &l.xv;
-      g.bias = which == 0 ? nullptr : l.xv_b;
-      g.x = d->enc;
-      g.ldx = D;
-      g.y = tmp;
-      g.ldy = D;
-      run_gemv_now(g, T, d->s);
-      if (which == 0 ? d->cross_i8k : d->cross_i8v)
+      const Mat &m = which == 0 ? l.xk : l.xv;
+      const float *bias = which == 0 ? nullptr : l.xv_b;
+      uint16_t *dst = which == 0 ? l.ck : l.cv;
+      const bool i8 = which == 0 ? d->cross_i8k : d->cross_i8v;
+      if (wide) {
+        WideGemm g;
+        g.wdtype = m.wdtype;
+        g.w = m.w;
+        g.scale = m.scale;
+        g.exps = m.exps;
+        g.bias = bias;
+        g.m = D;
+        g.k = D;
+        g.n = T;
+        g.rows = rows;
+        if (i8) {
+          g.y = tmp;
+          g.ldy = D;
+        } else {  // straight into the cache
+          g.pack = dst;
+          g.pack_hd = c.head_dim;
+          g.pack_t = T;
+        }
+        launch_wide_gemm(g, d->s);
+      } else {
+        GemvCall g;
+        g.m = &m;
+        g.bias = bias;
+        g.x = d->enc;
+        g.ldx = D;
+        g.y = tmp;
+        g.ldy = D;
+        run_gemv_now(g, T, d->s);
+      }
+      if (i8)
         hipLaunchKernelGGL(cross_quant_kernel, dim3(c.n_heads), dim3(256), 0, d->s, tmp, T, c.n_heads, c.head_dim,
-                           reinterpret_cast<int8_t *>(which == 0 ? l.ck : l.cv), which == 0 ? l.cks : l.cvs);
-      else
-        hipLaunchKernelGGL(cross_pack_kernel, dim3(1024), dim3(256), 0, d->s, tmp, T, c.n_heads,
-                           c.head_dim, which == 0 ? l.ck : l.cv);
+                           reinterpret_cast<int8_t *>(dst), which == 0 ? l.cks : l.cvs);
+      else if (!wide)
+        hipLaunchKernelGGL(cross_pack_kernel, dim3(1024), dim3(256), 0, d->s, tmp, T, c.n_heads, c.head_dim, dst);
       XE_HIP(hipGetLastError());
     }
   }

@@ -72,10 +72,10 @@ def prompt_cfg(xe, family, wd):
 
 
 @pytest.mark.parametrize("family,wd,batch,n", [
-    ("gemma", "i8", 1, 4), ("gemma", "i8", 1, 65), ("gemma", "i8", 1, 66), ("gemma", "bf16", 3, 50),
-    ("gemma", "i8", 2, 330), ("gemma_hd128", "i8", 2, 70), ("gemma", "bfp16", 22, 4),
+    ("gemma", "i8", 1, 4), ("gemma", "i8", 1, 129), ("gemma", "i8", 1, 130), ("gemma", "bf16", 3, 50),
+    ("gemma", "i8", 2, 3), ("gemma", "i8", 2, 330), ("gemma_hd128", "i8", 2, 70), ("gemma", "bfp16", 22, 4),
     ("opt", "i8", 1, 70), ("opt", "bfp16", 5, 40), ("opt", "i8", 20, 111),
-    ("whisper", "i8", 1, 5), ("whisper", "i8", 7, 29), ("whisper", "bf16", 3, 80)])
+    ("opt", "bf16", 3, 66), ("whisper", "i8", 1, 5), ("whisper", "bfp16", 7, 29), ("whisper", "bf16", 3, 80)])
 def test_prompt_passes_logits(gpu, xe, family, wd, batch, n):
     cfg = prompt_cfg(xe, family, wd)
     print("[case] prompt %s %s batch %d, %d tokens" % (family, wd, batch, n), flush=True)

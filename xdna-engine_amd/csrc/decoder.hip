@@ -1797,7 +1797,11 @@ void run_gemv_now(const GemvCall &g, int batch, hipStream_t s) {
 // prompt runs in chunks of tokens); the weights are read once a pass instead
 // of once a token.
 constexpr int kPromptRows = 2048;
-constexpr int kPromptWideRows = 65;
+// Rows from which the projections run on the plane kernels (wide.hip).  Whole
+// passes of Gemma-3-1B, ms here / with the decode step's GEMM: 64 rows 2.15 /
+// 1.90, 65 to 128 rows 2.40 / 2.38 to 2.52 / 2.47, 192 rows 3.02 / 3.17, 512
+// rows 4.35 / 5.88.
+constexpr int kPromptWideRows = 129;
 
 // Device workspace of a prompt pass of up to `rows` rows, one allocation.
 struct PromptWs {
@@ -2033,7 +2037,10 @@ void prompt_chunk(xe_decoder *d, const PromptWs &w, int B, int t0, int t_n, bool
 bool prompt_in_passes(xe_decoder *d, int batch, int n_prompt) {
   const auto &c = d->c;
   if (d->cross_i8k || d->cross_i8v) return false;  // int8 cross rows: the single-query kernels read them
-  return n_prompt >= 3 && batch <= kPromptRows && prompt_attn_takes(c.head_dim, c.n_heads / c.n_kv_heads);
+  // a pass of a few rows takes about two decode steps' time (Gemma-3-1B: 1.4
+  // ms for 4 to 16 rows, 0.77 a step at one stream, 1.5 to 2 beyond four;
+  // OPT-125m 0.57 / 0.3), under four rows on the GEMV a little more
+  return (n_prompt >= 3 || (n_prompt == 2 && batch >= 2)) && batch <= kPromptRows && prompt_attn_takes(c.head_dim, c.n_heads / c.n_kv_heads);
 }
 
 // The prompt in passes over up to kPromptRows rows; h: pinned staging.

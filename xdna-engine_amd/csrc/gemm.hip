@@ -1464,7 +1464,7 @@ size_t gemm_op_cnt_words() { return kGemmMaxTiles; }
 namespace {
 bool op_wide(const GemvLaunch &L) {
   return L.act == ACT_NONE && !L.sub && !L.res_out && L.out_scale == 1.0f &&
-         wide_preferred(L.m, L.k, L.batch) && wide_takes(L.m, L.k, L.batch, L.wdtype, L.x, L.ldx);
+         wide_preferred(L.m, L.k, L.batch, L.wdtype, gemm_needs_prologue(gdev::to_params(L))) && wide_takes(L.m, L.k, L.batch, L.wdtype, L.x, L.ldx);
 }
 }  // namespace
 

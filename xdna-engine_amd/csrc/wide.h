@@ -57,8 +57,8 @@ struct WideGemm {
 // Whether the shapes, sizes and alignments suit these kernels.
 bool wide_takes(int m, int k, int n, int wdtype, const void *x, int ldx);
 // Whether a linear of n rows over an m x k weight is faster here than on the
-// kernels of gemm.hip.
-bool wide_preferred(int m, int k, int n);
+// kernels of gemm.hip (prologue: those need one too).
+bool wide_preferred(int m, int k, int n, int wdtype, bool prologue);
 // K splits wide_gemm takes for a shape, with at most ws_floats floats of partials.
 int wide_splits(int m, int k, int n, int wdtype, size_t ws_floats);
 // x (+ sub, post norm, norm) of n rows -> planes; the fields x, x_bf16, ldx,

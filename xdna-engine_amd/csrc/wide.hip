@@ -32,9 +32,10 @@ typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kT = 256;
 constexpr int kBK = 64;             // k per step
@@ -42,6 +43,7 @@ constexpr int kNoRec = 0x7ffffff0;  // past every buffer: loads return zeros
 constexpr int kMaxK = 16384;        // rows kernel: 16 float4 a thread
 constexpr int kMaxKs = 8;           // K splits
 constexpr int kRowPad = 128;        // rexp is readable up to a multiple of it
+constexpr int kLds = 160 * 1024;    // LDS of a CU
 
 template <int WT>
 constexpr int planes_of() {
@@ -246,8 +248,22 @@ struct WideParams {
   int pack_hd, pack_t;
   float *part;
   int spk;       // steps a split
+  int vec;       // the output rows take 16-byte stores
   int tx, tw;    // row tiles, weight tiles
 };
+
+// gelu_tanh(x) = x / 2 (1 + tanh u) = x / (1 + exp(-2 u)): the same function
+// without the cancellation of 1 + tanh u, and a tenth of tanhf's instructions
+// (a big tile's 64 outputs a thread: 6 us of its epilogue).
+__device__ __forceinline__ float gelu_tanh_wide(float x) {
+  const float u2 = 2.0f * 0.79788456f * (x + 0.044715f * x * x * x);
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * u2));
+}
+
+// LDS offset of the epilogue's tables: behind the operand buffers and the
+// waves' output areas (which overlap).
+constexpr int epi_offset(int buffers, int out) { return ((buffers > out ? buffers : out) + 15) / 16 * 16; }
+constexpr int epi_tables(int bx, int bw) { return 4 * (bx + 2 * bw); }
 
 template <int WT>
 struct WTraits {
@@ -311,11 +327,11 @@ __device__ __forceinline__ bf16x8 bfp_to_bf16(uint32_t q0, uint32_t q1, uint32_t
 }
 
 template <int WT>
-__device__ __forceinline__ f32x16 mfma(u32x4 x, u32x4 w, f32x16 c) {
+__device__ __forceinline__ f32x16 mfma(u32x4 w, u32x4 x, f32x16 c) {
   if constexpr (WT == XE_I8 || WT == XE_I4)
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, x), __builtin_bit_cast(f16x8, w), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, x), c, 0, 0, 0);
   else
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, x), __builtin_bit_cast(bf16x8, w), c, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w), __builtin_bit_cast(bf16x8, x), c, 0, 0, 0);
 }
 
 // Tile: 32 RX WXN rows x 32 RW WWN weight rows a workgroup of WXN x WWN waves
@@ -324,8 +340,10 @@ __device__ __forceinline__ f32x16 mfma(u32x4 x, u32x4 w, f32x16 c) {
 // step; the loads of NS steps are in flight), and come back as
 // v_mfma_f32_32x32x16 operands: lane half h takes k 32 h .. + 31 of the step,
 // 8 of them a MFMA, the same for rows and weights; weights convert to 16 bits
-// after the LDS read.  The row operand is A, so a lane's results are 16 rows
-// of one weight row: 32 lanes store 32 neighbouring outputs.
+// after the LDS read.  The weight operand is A, so a lane's results are
+// quads of neighbouring outputs of one row; the wave turns them through LDS
+// and stores whole row segments, 16 bytes a lane (4-byte stores straight from
+// the accumulators took 7 to 10 us of a 48 us launch at 13824 x 1152 x 512).
 // Workgroups are numbered so that the row tiles of one weight tile run on one
 // XCD, one after the other: its weights are read from HBM once.
 template <int WT, int WXN, int WWN, int RX, int RW, int NS, int NB>
@@ -336,6 +354,12 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
   constexpr int ROWB = WTraits<WT>::kRowB;
   constexpr int XB = P * BX * 128, WB = BW * ROWB, EB = WT == XE_BFP16 ? BW * 8 : 0;
   constexpr int BUF = XB + WB + EB;
+  constexpr int OS = 32 * RW + 4;                             // row stride (floats) of a wave's output area
+  constexpr int OB = 32 * RX * OS * 4;                        // its bytes, over the operand buffers after the K loop
+  constexpr int kTab = epi_tables(BX, BW);
+  // the tables go in before the K loop where they fit behind its buffers
+  constexpr bool kEarly = epi_offset(NB * BUF, WXN * WWN * OB) + kTab <= kLds;
+  constexpr int kEpi = epi_offset(kEarly ? NB * BUF : 0, WXN * WWN * OB);
   constexpr int NX = P * BX * 8 / T;                          // 16-byte row chunks a thread
   constexpr int NW = (WT == XE_BF16 ? BW * 8 : BW * 4) / T;   // weight chunks a thread
   constexpr int PA = RX * RW == 1 ? P : 1;                    // accumulators a block (independent MFMA chains)
@@ -400,18 +424,6 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
         st.e[j] = __builtin_amdgcn_raw_buffer_load_b16(re, wok ? eoff[j] : kNoRec, k0 / 8, 0);
     }
   };
-  // what the epilogue needs, loaded now: the rows' exponents (LDS, behind the
-  // operand buffers) and this lane's weight rows' scales and biases
-  int *const rs = reinterpret_cast<int *>(lds + NB * BUF);
-  if constexpr (P == 2)
-    if (threadIdx.x < BX) rs[threadIdx.x] = p.rexp[n0 + threadIdx.x];
-  float sc[RW], bi[RW];
-#pragma unroll
-  for (int b = 0; b < RW; b++) {
-    const int m = min(m0 + ww * 32 * RW + 32 * b + (lane & 31), p.m - 1);
-    sc[b] = !p.part && (WT == XE_I8 || WT == XE_I4) ? p.scale[m] : 1.0f;
-    bi[b] = !p.part && p.bias ? p.bias[m] : 0.0f;
-  }
   const int xput = lds_chunk<128>(xr, xc);
   const int wput = WT == XE_I4 ? lds_chunk<32>(wr, wc >> 1) + 8 * (wc & 1) : lds_chunk<ROWB>(wr, wc);
   auto put = [&](int buf, const Stage &st) {
@@ -498,7 +510,6 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
         rdx(bn, 0, 0);
         rdq(bn, q[(j + 1) % QN], ex[(j + 1) % QN]);
       }
-      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int b = 0; b < RW; b++) {
         if constexpr (WT == XE_I8) wf[s & 1][b] = __builtin_bit_cast(u32x4, i8_to_f16(qv[b][2 * s], qv[b][2 * s + 1]));
@@ -512,12 +523,11 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
         for (int a = 0; a < RX; a++)
 #pragma unroll
           for (int b = 0; b < RW; b++)
-            acc[a][b][pl % PA] = mfma<WT>(xf[s & 1][a][pl], wf[s & 1][b], acc[a][b][pl % PA]);
+            acc[a][b][pl % PA] = mfma<WT>(wf[s & 1][b], xf[s & 1][a][pl], acc[a][b][pl % PA]);
       if (s == 0) {
         put(bp, sj);
         if constexpr (decltype(more)::value) issue(next_issue, sj);
       }
-      __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();
     bc = bn;
@@ -525,6 +535,26 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
   };
 #pragma unroll
   for (int j = 0; j < NS; j++) issue(j, st[j]);
+  // what the epilogue needs, loaded behind the first operands, in LDS: the
+  // rows' exponents, the weight rows' scales and biases
+  int *const rs = reinterpret_cast<int *>(lds + kEpi);
+  float *const wsc = reinterpret_cast<float *>(rs + BX), *const wbi = wsc + BW;
+  int t_rs = 0;
+  float t_sc = 1.0f, t_bi = 0.0f;
+  if constexpr (P == 2) t_rs = p.rexp[n0 + threadIdx.x % BX];
+  {
+    const int m = min(m0 + static_cast<int>(threadIdx.x) % BW, p.m - 1);
+    if constexpr (WT == XE_I8 || WT == XE_I4) t_sc = p.scale[m];
+    if (p.bias) t_bi = p.bias[m];
+  }
+  auto put_tables = [&]() {
+    if (threadIdx.x < BX) rs[threadIdx.x] = t_rs;
+    if (threadIdx.x < BW) {
+      wsc[threadIdx.x] = t_sc;
+      wbi[threadIdx.x] = t_bi;
+    }
+  };
+  if constexpr (kEarly) put_tables();
 #pragma unroll
   for (int d = 0; d < D; d++) {
     put(d * BUF, st[d % NS]);
@@ -546,65 +576,74 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
   for (int j = 0; j < NS - 1; j++)
     if (s0 + j < nsteps) step(j, 0, std::false_type{});
 
-  // a lane's results: rows 8 (i / 4) + 4 (lane / 32) + i % 4 of weight row lane % 32
+  // A lane's results: weight rows 8 (i / 4) + 4 (lane / 32) + i % 4 of row
+  // lane % 32 of each block.  The epilogue in registers, then through the
+  // wave's own LDS area (the operand buffers are free since the last barrier)
+  // into stores along the rows.
+  if constexpr (!kEarly) {
+    put_tables();
+    __syncthreads();
+  }
+  float *const out = reinterpret_cast<float *>(lds + wave * OB);
+  const bool geglu = p.act == ACT_GEGLU_TANH && !p.part;
 #pragma unroll
-  for (int b = 0; b < RW; b++) {
-    const int m = m0 + ww * 32 * RW + 32 * b + lr;
+  for (int a = 0; a < RX; a++) {
+    int sx = 0;
+    if constexpr (P == 2) sx = -rs[wx * 32 * RX + 32 * a + lr];
+    float *const orow = out + (32 * a + lr) * OS;
 #pragma unroll
-    for (int a = 0; a < RX; a++) {
-      const int nb = n0 + wx * 32 * RX + 32 * a + 4 * lh;
+    for (int b = 0; b < RW; b++)
 #pragma unroll
       for (int i4 = 0; i4 < 4; i4++) {
-        const int n = nb + 8 * i4;
+        const int ml = 32 * b + 8 * i4 + 4 * lh;
         float v[4];
-        i32x4 s4 = {0, 0, 0, 0};
-        if constexpr (P == 2) s4 = *reinterpret_cast<const i32x4 *>(rs + (n - n0));
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           float t = acc[a][b][0][4 * i4 + i];
 #pragma unroll
           for (int q = 1; q < PA; q++) t += acc[a][b][q][4 * i4 + i];
-          if constexpr (P == 2) t = __builtin_ldexpf(t, -s4[i]);
+          if constexpr (P == 2) t = __builtin_ldexpf(t, sx);
           v[i] = t;
         }
-        if (p.part) {
-          if (m < p.m)
+        if (!p.part) {
+          const f32x4 sc = *reinterpret_cast<const f32x4 *>(wsc + ww * 32 * RW + ml);
+          const f32x4 bi = *reinterpret_cast<const f32x4 *>(wbi + ww * 32 * RW + ml);
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-              if (n + i < p.n) p.part[(static_cast<size_t>(z) * p.n + n + i) * p.m + m] = v[i];
-          continue;
-        }
+          for (int i = 0; i < 4; i++) v[i] = v[i] * sc[i] + bi[i];
+          if (p.act == ACT_RELU) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = v[i] * sc[b] + bi[b];
-        if (p.act == ACT_GEGLU_TANH) {
-          // lanes 2 r (gate) and 2 r + 1 (up): the even lane finishes rows
-          // n, n + 2, the odd lane rows n + 1, n + 3
-          const bool odd = lane & 1;
+            for (int i = 0; i < 4; i++) v[i] = v[i] > 0.f ? v[i] : 0.f;
+          } else if (p.act == ACT_GELU_ERF) {
 #pragma unroll
-          for (int i = 0; i < 4; i += 2) {
-            const float send = odd ? v[i] : v[i + 1];
-            const float got = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(send), 0xB1, 0xf, 0xf, true));
-            const float gate = odd ? got : v[i], up = odd ? v[i + 1] : got;
-            const int nn = n + i + (odd ? 1 : 0);
-            if (m < p.m && nn < p.n) p.y[static_cast<size_t>(nn) * p.ldy + (m >> 1)] = gdev::gelu_tanh(gate) * up;
-          }
-        } else if (p.pack) {
-          if (m < p.m) {
-            const size_t o = static_cast<size_t>(m / p.pack_hd) * p.pack_t * p.pack_hd + m % p.pack_hd;
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-              if (n + i < p.n) p.pack[o + static_cast<size_t>(n + i) * p.pack_hd] = adev::f32_to_bf16_rne(v[i]);
-          }
-        } else if (m < p.m) {
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            float t = v[i];
-            if (p.act == ACT_RELU) t = t > 0.f ? t : 0.f;
-            else if (p.act == ACT_GELU_ERF) t = gdev::gelu_erf(t);
-            if (n + i < p.n) p.y[static_cast<size_t>(n + i) * p.ldy + m] = t;
+            for (int i = 0; i < 4; i++) v[i] = gdev::gelu_erf(v[i]);
           }
         }
+        if (geglu)  // weight rows 2 r (gate) and 2 r + 1 (up)
+          *reinterpret_cast<f32x2 *>(orow + ml / 2) = f32x2{gelu_tanh_wide(v[0]) * v[1], gelu_tanh_wide(v[2]) * v[3]};
+        else
+          *reinterpret_cast<f32x4 *>(orow + ml) = f32x4{v[0], v[1], v[2], v[3]};
       }
+  }
+  // the wave's rows: CQ quads each
+  const int cq = geglu ? 4 * RW : 8 * RW, cols = geglu ? p.m / 2 : p.m;
+  const int c0 = (m0 + ww * 32 * RW) / (geglu ? 2 : 1);
+  const int ld = p.part ? p.m : p.ldy;
+  float *const y = p.part ? p.part + static_cast<size_t>(z) * p.n * p.m : p.y;
+  for (int id = lane; id < 32 * RX * cq; id += 64) {
+    const int r = id / cq, c = 4 * (id % cq);
+    const int n = n0 + wx * 32 * RX + r, m = c0 + c;
+    if (n >= p.n || m >= cols) continue;
+    const f32x4 v = *reinterpret_cast<const f32x4 *>(out + r * OS + c);
+    if (p.pack && !p.part) {
+      const uint32_t lo = adev::f32_to_bf16_rne(v.x) | static_cast<uint32_t>(adev::f32_to_bf16_rne(v.y)) << 16;
+      const uint32_t hi = adev::f32_to_bf16_rne(v.z) | static_cast<uint32_t>(adev::f32_to_bf16_rne(v.w)) << 16;
+      *reinterpret_cast<u32x2 *>(p.pack + (static_cast<size_t>(m / p.pack_hd) * p.pack_t + n) * p.pack_hd + m % p.pack_hd) = u32x2{lo, hi};
+    } else if (p.vec) {
+      *reinterpret_cast<f32x4 *>(y + static_cast<size_t>(n) * ld + m) = v;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (m + i < cols) y[static_cast<size_t>(n) * ld + m + i] = v[i];
     }
   }
 }
@@ -651,8 +690,8 @@ __global__ __launch_bounds__(kT) void wide_finish_kernel(WideParams p, int ks, i
   }
   if constexpr (V == 4)
     if (p.act == ACT_GEGLU_TANH) {
-      p.y[static_cast<size_t>(n) * p.ldy + m / 2] = gdev::gelu_tanh(v[0]) * v[1];
-      p.y[static_cast<size_t>(n) * p.ldy + m / 2 + 1] = gdev::gelu_tanh(v[2]) * v[3];
+      p.y[static_cast<size_t>(n) * p.ldy + m / 2] = gelu_tanh_wide(v[0]) * v[1];
+      p.y[static_cast<size_t>(n) * p.ldy + m / 2 + 1] = gelu_tanh_wide(v[2]) * v[3];
     }
 }
 
@@ -661,38 +700,39 @@ __global__ __launch_bounds__(kT) void wide_finish_kernel(WideParams p, int ks, i
 //          of the small tile; one workgroup a CU
 //   small  64 x 64, 4 waves, loads of four steps in flight: shapes whose big
 //          tiles leave CUs idle
-// Cost in microseconds, fitted to launches over one dimension at a time
-// (512 rows, int8 / bf16 weights): a big tile's step takes 1.47 / 2.13 us
-// (68 % of the matrix rate) and its launch 8 us of latency; a small tile's
-// 0.44 / 0.72 us, alone on its CU or 1.25 times that for each workgroup of
-// it; a K split writes and reads its partials at about 4 TB/s.
+// Cost in microseconds, fitted to launches over one dimension at a time (512
+// rows, int8 / bf16 weights): a big tile's step takes 1.27 / 1.83 us (64 to 67
+// % of the matrix cores' cycles) and its launch 6 us of latency; a small
+// tile's 0.44 / 0.58 us, alone on its CU or 1.25 times that for each
+// workgroup of it; a K split writes and reads its partials at about 4 TB/s.
 struct Shape {
   bool big;
   int ks, spk;
 };
 constexpr int kTileX[2] = {64, 128}, kTileW[2] = {64, 256};
 
-Shape choose_shape(int m, int k, int n, int wdtype, size_t ws_floats) {
+Shape choose_shape(int m, int k, int n, int wdtype, size_t ws_floats, double *cost_us = nullptr) {
   const int steps = (k + kBK - 1) / kBK;
-  const int planes = wide_planes(wdtype);
+  const bool p2 = wide_planes(wdtype) == 2;
   Shape best{false, 1, steps};
   double best_cost = -1;
   for (int big = 0; big < 2; big++) {
     const long tiles = static_cast<long>((m + kTileW[big] - 1) / kTileW[big]) * ((n + kTileX[big] - 1) / kTileX[big]);
-    const double step = big ? (planes == 2 ? 1.47 : 2.2) : (planes == 2 ? 0.44 : 0.7);
+    const double step = big ? (p2 ? 1.27 : 1.83) : (p2 ? 0.44 : 0.58);
     for (int ks = 1; ks <= kMaxKs; ks++) {
       const int spk = (steps + ks - 1) / ks;
       if ((steps + spk - 1) / spk != ks) continue;
       if (ks > 1 && (spk < 4 || static_cast<size_t>(ks) * n * m > ws_floats)) continue;
       const double wgs = static_cast<double>(tiles) * ks / 256.0;
-      double cost = big ? 8.0 + spk * step * std::ceil(wgs) : 4.0 + spk * step * std::max(1.0, 1.25 * wgs);
-      if (ks > 1) cost += 3.0 + static_cast<double>(ks) * n * m * 2e-6;  // partials out and back
+      double cost = big ? 6.0 + spk * step * std::ceil(wgs) : 3.0 + spk * step * std::max(1.0, 1.25 * wgs);
+      if (ks > 1) cost += 3.0 + static_cast<double>(ks) * n * m * 2e-6;
       if (best_cost < 0 || cost < best_cost) {
         best_cost = cost;
         best = {big != 0, ks, spk};
       }
     }
   }
+  if (cost_us) *cost_us = best_cost;
   return best;
 }
 
@@ -708,8 +748,10 @@ WideFn pick(bool big) {
 
 int lds_bytes(int wdtype, bool big) {
   const int bx = kTileX[big], bw = kTileW[big], rowb = wdtype == XE_BF16 ? 128 : wdtype == XE_I4 ? 32 : 64;
-  return buffers(wdtype) * (wide_planes(wdtype) * bx * 128 + bw * rowb + (wdtype == XE_BFP16 ? bw * 8 : 0)) +
-         (wide_planes(wdtype) == 2 ? 4 * bx : 0);
+  const int bufs = buffers(wdtype) * (wide_planes(wdtype) * bx * 128 + bw * rowb + (wdtype == XE_BFP16 ? bw * 8 : 0));
+  const int out = big ? 8 * 64 * 68 * 4 : 4 * 32 * 36 * 4;  // the waves' output areas
+  const int early = epi_offset(bufs, out) + epi_tables(bx, bw);
+  return early <= kLds ? early : std::max(bufs, epi_offset(0, out) + epi_tables(bx, bw));
 }
 
 template <int P>
@@ -737,11 +779,20 @@ bool wide_takes(int m, int k, int n, int wdtype, const void *x, int ldx) {
          wide_plane_elems(wdtype, n + kRowPad, k) * 2 < (size_t(1) << 31);
 }
 
-// From about 3.5 G multiply-adds on; below, the kernels of gemm.hip, which
-// need no planes, are as fast or faster (us, int8: 4096 x 4096 at 200 rows 43
-// here, 43 there; 1152 x 6912 at 512 rows 52 / 64; 1152 x 1152 at 512 rows
-// 19 / 17; 768 x 3072 at 100 rows 17 / 12).
-bool wide_preferred(int m, int k, int n) { return n > 64 && static_cast<double>(m) * k * n >= 3.5e9; }
+// The rows kernel and its launch take about 6 us; the kernels of gemm.hip,
+// which need no planes but split the rows in every weight tile, 8 us and 11.5
+// us for every 1e9 multiply-adds (int8 and bf16 alike), after a prologue of 5
+// us for a norm.  Measured here / there, us: int8 1152 x 1152 at 512 rows 18.5
+// / 16.6, 3072 x 768 at 512 19.9 / 24.4, 4096 x 4096 at 200 36 / 40, 1152 x
+// 6912 at 512 50 / 64, 13824 x 1152 at 512 47 / 107, 14336 x 4096 at 512 121 /
+// 342; bf16 3072 x 768 at 512 28 / 23.5, 4096 x 4096 at 200 40 / 40 (where the
+// estimates are within 5 % the other kernels stay).
+bool wide_preferred(int m, int k, int n, int wdtype, bool prologue) {
+  if (n <= 64) return false;  // one stream tile of gemm.hip
+  double us = 0;
+  (void)choose_shape(m, k, n, wdtype, gemm_op_ws_floats(), &us);
+  return us + 6.0 + 2e-6 * n * k < 0.95 * (8.0 + 11.5e-9 * m * static_cast<double>(k) * n + (prologue ? 5.0 : 0.0));
+}
 
 int wide_splits(int m, int k, int n, int wdtype, size_t ws_floats) {
   return choose_shape(m, k, n, wdtype, ws_floats).ks;
@@ -767,6 +818,7 @@ void launch_wide_gemm(const WideGemm &g, hipStream_t s) {
   XE_REQUIRE((g.wdtype != XE_I8 && g.wdtype != XE_I4) || (g.scale && g.rows.rexp), "wide gemm: int8/int4 weight without scales");
   XE_REQUIRE(g.wdtype != XE_BFP16 || g.exps, "wide gemm: bfp16 weight without exponents");
   XE_REQUIRE(g.act != ACT_GEGLU_TANH || (g.m % 4 == 0 && !g.pack), "wide gemm: GeGLU rows must pair within 4-row groups");
+  XE_REQUIRE(!g.pack || (g.m % g.pack_hd == 0 && g.pack_hd % 4 == 0), "wide gemm: packed heads must hold whole quads");
   const size_t ws = g.part || g.ws ? g.ws_floats : 0;
   const Shape sh = choose_shape(g.m, g.k, g.n, g.wdtype, ws);
   XE_REQUIRE(!g.part || sh.ks > 1, "wide gemm: partials of an unsplit product");
@@ -788,6 +840,8 @@ void launch_wide_gemm(const WideGemm &g, hipStream_t s) {
   p.pack_t = g.pack_t;
   p.part = sh.ks > 1 ? (g.part ? g.part : g.ws) : nullptr;
   p.spk = sh.spk;
+  const int cols = g.act == ACT_GEGLU_TANH && !p.part ? g.m / 2 : g.m;
+  p.vec = cols % 4 == 0 && (p.part ? al16(p.part) : al16(g.y) && g.ldy % 4 == 0);
   p.tx = (g.n + kTileX[sh.big] - 1) / kTileX[sh.big];
   p.tw = (g.m + kTileW[sh.big] - 1) / kTileW[sh.big];
   WideFn fn = nullptr;

@@ -1,0 +1,39 @@
+"""Split attention whose partials merge in groups: split counts either side of
+one group (16 splits), of groups of eight (up to 64) and of sixteen, streams
+of one split beside streams of many, against the oracle; and the merge inside
+the split kernel equal to the separate merge launch bit for bit."""
+import math
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from test_attn_gpu import close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("hq,hkv,hd,ctxlen,b", [
+    (4, 1, 256, 1024, 1), (4, 1, 256, 1088, 1), (4, 1, 256, 4096, 3), (4, 1, 256, 4160, 2), (4, 1, 256, 16384, 1),
+    (2, 2, 64, 3000, 5), (8, 1, 128, 9000, 2), (12, 12, 64, 2100, 1)])
+def test_grouped_merge(gpu, monkeypatch, hq, hkv, hd, ctxlen, b):
+    _, ctx = gpu
+    print("[case] grouped merge hq=%d hkv=%d hd=%d ctx=%d b=%d" % (hq, hkv, hd, ctxlen, b), flush=True)
+    rng = np.random.default_rng(hq + hd + ctxlen + b)
+    lens = rng.integers(1, ctxlen + 1, b).astype(np.int32)
+    lens[0] = ctxlen
+    if b > 1:
+        lens[1] = 3
+    q = rng.standard_normal((b, hq, hd)).astype(np.float32)
+    kc = O.bf16_bits(rng.standard_normal((b, hkv, ctxlen, hd)).astype(np.float32))
+    vc = O.bf16_bits(rng.standard_normal((b, hkv, ctxlen, hd)).astype(np.float32))
+    scale = 1.0 / math.sqrt(hd)
+    first = ctx.attn(q, kc, vc, lens, scale)
+    again = ctx.attn(q, kc, vc, lens, scale)  # the arrival counters are zero again
+    monkeypatch.setenv("XE_ATTN_MERGE", "launch")
+    launched = ctx.attn(q, kc, vc, lens, scale)
+    monkeypatch.delenv("XE_ATTN_MERGE")
+    bits = np.asarray(first, np.float32).view(np.uint32)
+    assert np.array_equal(bits, np.asarray(again, np.float32).view(np.uint32))
+    assert np.array_equal(bits, np.asarray(launched, np.float32).view(np.uint32))
+    close(first, O.attn_decode(q, kc, vc, lens, scale))

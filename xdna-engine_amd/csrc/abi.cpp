@@ -845,7 +845,7 @@ int xe_w8a8_linear(xe_ctx *ctx, const xe_weight *w, const float *x, int batch, f
 }
 
 // Splits per (stream, kv head): about XE_ATTN_WG_PER_CU (default 2)
-// workgroups per CU in total, at most one per 64 cache rows and at most 64.
+// workgroups per CU in total, at most one per 64 cache rows and at most 256.
 // With the merge inside the split kernel, 2 a CU against 4 (graph replays,
 // config 3): GQA 4q/1kv x 256 b = 64 ctx 4096 52.3 / 58.3 us, b = 16 ctx
 // 4096 33.0 / 47.1, b = 64 ctx 1024 26.2 / 37.2; ctx 32768 within 4 %.
@@ -859,7 +859,7 @@ static int attn_splits(const xe_ctx *ctx, int batch, int hkv, int max_ctx) {
   const int cap = (max_ctx + 63) / 64;
   ms = ms < 1 ? 1 : ms;
   ms = ms > cap ? cap : ms;
-  return ms > 64 ? 64 : ms;
+  return ms > 256 ? 256 : ms;
 }
 
 // work: the split partials (attn_work_floats(batch, hq, hd, splits) floats);
@@ -895,7 +895,7 @@ static int attn_impl(xe_ctx *ctx, const float *q, const uint16_t *kc, const uint
   } else {
     const bool in_place = attn_merge_in_place();
     ctx->ensure_attn(attn_work_floats(batch, hq, hd, a.max_splits),
-                     in_place ? static_cast<size_t>(batch) * hkv : 0);
+                     in_place ? attn_cnt_words(batch, hkv) : 0);
     a.work = ctx->attn_work;
     a.cnt = in_place ? ctx->attn_cnt : nullptr;
   }
@@ -1095,7 +1095,7 @@ int xe_probe_attn(xe_ctx *ctx, const float *q_dev, const uint16_t *kc_dev, const
     XE_REQUIRE(batch > 0 && hq > 0 && hkv > 0 && hd > 0 && reps > 0, "bad shape");
     DeviceGuard dg(ctx->dev->ordinal);
     ctx->ensure_attn(attn_work_floats(batch, hq, hd, attn_splits(ctx, batch, hkv, max_ctx)),
-                     attn_merge_in_place() ? static_cast<size_t>(batch) * hkv : 0);  // no allocation under capture
+                     attn_merge_in_place() ? attn_cnt_words(batch, hkv) : 0);  // no allocation under capture
     *us_per_call = time_captured(ctx, reps, flags, [&]() {
       attn_impl(ctx, q_dev, kc_dev, vc_dev, lens_dev, batch, hq, hkv, hd, max_ctx, scale, out_dev);
     });

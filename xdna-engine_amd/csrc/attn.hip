@@ -130,6 +130,8 @@ void launch_attn_phase(const sdev::Phase &ph, hipStream_t s) {
   XE_HIP(hipGetLastError());
 }
 
+size_t attn_cnt_words(int batch, int hkv) { return static_cast<size_t>(batch) * hkv * adev::kCntWords; }
+
 size_t attn_work_floats(int batch, int hq, int hd, int max_splits) {
   return static_cast<size_t>(batch) * hq * max_splits * (hd + 2);
 }

@@ -24,8 +24,9 @@
 // without counters).  With arrival counters (AttnParams::cnt) the split
 // kernel merges in place instead: each split block stores
 // its partial with sc1 stores (past the XCD's own L2), waits for them, counts
-// itself in the (stream, kv head)'s counter with an agent-scope atomic, and
-// the last to arrive reads every partial with sc1 loads and writes the output
+// itself in its counter with an agent-scope atomic, and the last to arrive
+// reads the partials with sc1 loads and writes the output (more than kGroup
+// splits: first its group's merged partial, then the last group the output)
 // (no device-scope release/acquire fences: those write back and invalidate L2
 // on this part and measured ~80 us per launch).
 // Fused in front (decode step): the Gemma per-head RMSNorm (1 + w) and RoPE of
@@ -48,6 +49,17 @@ constexpr int kWaves = 4;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kMinChunk = 64;  // keys per split at least (amortises per-block setup)
 constexpr int kMaxSplits = 256;
+// Split partials merge in groups of kGroup, then the groups: one merging
+// block reads at most kGroup partials, so a long context of few streams can
+// split over the whole chip.  4 heads x 256, one key head, us, all splits (64
+// at most) merged by one block / in groups: 32768 keys of one stream 47.4 /
+// 25.5 (256 splits), 4096 keys of one 29.3 / 16.0, of 8 streams 32.6 / 19.5.
+constexpr int kGroup = 16;  // partials a merge takes, and groups
+static_assert(kGroup * kGroup >= kMaxSplits, "two levels of groups cover every split count");
+constexpr int kCntWords = 1 + kGroup;  // arrival counters of a (stream, kv head)
+// Splits a group: all of them up to kGroup; up to 64 in eights (either level
+// of the merge is one load round trip), beyond in sixteens.
+__device__ __forceinline__ int group_size(int nsplits) { return nsplits <= 64 && nsplits > kGroup ? 8 : kGroup; }
 
 using gdev::act_ld;
 using gdev::act_st;
@@ -75,8 +87,8 @@ struct AttnParams {
   float *work;
   int max_splits;
   const float *k_scale, *v_scale;  // int8 K / V channel scales [hkv * hd], or null (bf16)
-  unsigned *cnt;  // [batch * hkv] arrival counters (zero between launches): merge in the
-                  // split kernel; null: a merge phase follows
+  unsigned *cnt;  // [batch * hkv][kCntWords] arrival counters (zero between launches): merge
+                  // in the split kernel; null: a merge phase follows
 };
 
 __device__ __forceinline__ uint16_t f32_to_bf16_rne(float x) {
@@ -110,7 +122,7 @@ __host__ __device__ constexpr size_t attn_lds_floats(int hd, int g) {
   return static_cast<size_t>(g) * hd + static_cast<size_t>(kWaves) * g * (hd + 2);
 }
 __host__ __device__ constexpr size_t merge_lds_floats() {
-  return static_cast<size_t>(4) * kMaxSplits + 4;
+  return static_cast<size_t>(4) * (kGroup + 2);
 }
 
 // Per-head RMSNorm (1+w) and RoPE on one head vector held by one wave:
@@ -202,62 +214,50 @@ struct Raw8 {
 };
 
 // Phase 1 of a merge, heads [g0, g0 + ng) of one (stream, kv head) (waves
-// over heads, lanes over splits): wts[hh][s] = exp2(m_s - M) with M the
-// largest m_s, lsum[hh] = sum_s l_s wts[hh][s].  wbase: the partials of the
-// (stream, kv head), head g's split s at (g * max_splits + s) * (HD + 2).
+// over heads, lanes over partials): of the n <= kGroup partials s0 + i * step,
+// wts[hh][i] = exp2(m_i - M) with M the largest m_i (mmax[hh]), lsum[hh] =
+// sum_i l_i wts[hh][i].  wbase: the partials of the (stream, kv head), head
+// g's split s at (g * max_splits + s) * (HD + 2).
 template <int HD, bool LDCOH>
-__device__ __forceinline__ void merge_weights(const AttnParams &p, const float *wbase, int nsplits, int g0, int ng,
-                                              float *wts, float *lsum) {
+__device__ __forceinline__ void merge_weights(const AttnParams &p, const float *wbase, int s0, int step, int n, int g0,
+                                              int ng, float *wts, float *lsum, float *mmax) {
   constexpr int RS = HD + 2;  // floats of one partial: m, l, acc[HD]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int hh = wave; hh < ng; hh += kWaves) {
-    const int row = (g0 + hh) * p.max_splits;
-    float ls = 0.f;
-    if (nsplits <= 64) {  // one split a lane: m and l in one round trip
-      const bool on = lane < nsplits;
-      const int src = (row + (on ? lane : 0)) * RS;
-      const float ms = act_ld<LDCOH>(wbase, src), lv = act_ld<LDCOH>(wbase, src + 1);
-      float mx = on ? ms : -INFINITY;
+    const bool on = lane < n;
+    const int src = ((g0 + hh) * p.max_splits + s0 + (on ? lane : 0) * step) * RS;
+    const float ms = act_ld<LDCOH>(wbase, src), lv = act_ld<LDCOH>(wbase, src + 1);
+    float mx = on ? ms : -INFINITY;
 #pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-      const float f = !on || ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
-      if (on) {
-        wts[hh * kMaxSplits + lane] = f;
-        ls = lv * f;
-      }
-    } else {
-      float mx = -INFINITY;
-      for (int sidx = lane; sidx < nsplits; sidx += 64) mx = fmaxf(mx, act_ld<LDCOH>(wbase, (row + sidx) * RS));
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-      for (int sidx = lane; sidx < nsplits; sidx += 64) {
-        const int src = (row + sidx) * RS;
-        const float ms = act_ld<LDCOH>(wbase, src);
-        const float f = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
-        wts[hh * kMaxSplits + sidx] = f;
-        ls += act_ld<LDCOH>(wbase, src + 1) * f;
-      }
+    for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    const float f = !on || ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
+    if (on) wts[hh * kGroup + lane] = f;
+    const float ls = wave_sum(on ? lv * f : 0.f);
+    if (lane == 0) {
+      lsum[hh] = ls;
+      mmax[hh] = mx;
     }
-    ls = wave_sum(ls);
-    if (lane == 0) lsum[hh] = ls;
   }
 }
 
-// Merges heads [g0, g0 + ng) of (stream b, kv head kvh) from the nsplits
-// partials: out = sum_s acc_s w_s / sum_s l_s w_s (even and odd splits summed
-// apart, in split order, then added).  A thread takes outputs threadIdx.x +
-// j * kThreads, j < NE (ng * HD <= NE * kThreads).  The acc values of splits
-// [0, 8) are loaded before phase 1, so with at most 8 splits the merge takes
-// one memory round trip.  LDCOH: sc1 loads of the partials; STCOH:
-// agent-scope output stores.  lds: ng * (kMaxSplits + 1) floats.
-template <int HD, int G, int NE, bool LDCOH, bool STCOH>
-__device__ __forceinline__ void merge_heads(const AttnParams &p, int kvh, int b, int nsplits, int g0, int ng,
+// Merges heads [g0, g0 + ng) of (stream b, kv head kvh) from the n <= kGroup
+// partials s0 + i * step (even and odd ones summed apart, in order, then
+// added).  FINAL: out = sum_i acc_i w_i / sum_i l_i w_i; else the merged
+// partial (m, l, acc) replaces partial s0.  A thread takes outputs
+// threadIdx.x + j * kThreads, j < NE (ng * HD <= NE * kThreads).  The acc
+// values of the first SC partials are loaded before phase 1, so up to that
+// many take one memory round trip.  LDCOH: sc1 loads (and partial stores);
+// STCOH: agent-scope output stores.  lds: ng * (kGroup + 2) floats, free again
+// on return.
+template <int HD, int G, int NE, bool LDCOH, bool STCOH, bool FINAL>
+__device__ __forceinline__ void merge_heads(const AttnParams &p, int kvh, int b, int s0, int step, int n, int g0, int ng,
                                             float *lds) {
   constexpr int RS = HD + 2;
-  constexpr int SC = 8;  // splits a thread holds in registers at once
-  float *wts = lds;                     // [ng][kMaxSplits]
-  float *lsum = lds + ng * kMaxSplits;  // [ng]
-  const float *wbase = p.work + (static_cast<size_t>(b) * p.hq + kvh * G) * p.max_splits * RS;
+  constexpr int SC = 8;  // partials a thread holds in registers at once
+  float *wts = lds;                  // [ng][kGroup]
+  float *lsum = lds + ng * kGroup;   // [ng]
+  float *mmax = lsum + ng;           // [ng]
+  float *wbase = p.work + (static_cast<size_t>(b) * p.hq + kvh * G) * p.max_splits * RS;
   int src[NE], hw[NE];
   bool ok[NE];
   float at0[NE], at1[NE], v[SC][NE];
@@ -266,31 +266,31 @@ __device__ __forceinline__ void merge_heads(const AttnParams &p, int kvh, int b,
     const int t = threadIdx.x + j * kThreads;
     ok[j] = t < ng * HD;
     const int hh = ok[j] ? t / HD : 0, e = t % HD;
-    src[j] = (g0 + hh) * p.max_splits * RS + 2 + e;
-    hw[j] = hh * kMaxSplits;
+    src[j] = ((g0 + hh) * p.max_splits + s0) * RS + 2 + e;
+    hw[j] = hh * kGroup;
     at0[j] = 0.f;
     at1[j] = 0.f;
   }
-  auto load = [&](int s0) {
+  auto load = [&](int i0) {
 #pragma unroll
     for (int u = 0; u < SC; u++)
 #pragma unroll
       for (int j = 0; j < NE; j++)
-        v[u][j] = ok[j] && s0 + u < nsplits ? act_ld<LDCOH>(wbase, src[j] + (s0 + u) * RS) : 0.f;
+        v[u][j] = ok[j] && i0 + u < n ? act_ld<LDCOH>(wbase, src[j] + (i0 + u) * step * RS) : 0.f;
   };
   load(0);
-  merge_weights<HD, LDCOH>(p, wbase, nsplits, g0, ng, wts, lsum);
+  merge_weights<HD, LDCOH>(p, wbase, s0, step, n, g0, ng, wts, lsum, mmax);
   __syncthreads();
-  for (int s0 = 0; s0 < nsplits; s0 += SC) {
-    if (s0) load(s0);
+  for (int i0 = 0; i0 < n; i0 += SC) {
+    if (i0) load(i0);
 #pragma unroll
     for (int u = 0; u < SC; u++) {
-      if (s0 + u >= nsplits) break;
+      if (i0 + u >= n) break;
 #pragma unroll
       for (int j = 0; j < NE; j++) {
         if (!ok[j]) continue;
-        if (u & 1) at1[j] += v[u][j] * wts[hw[j] + s0 + u];
-        else at0[j] += v[u][j] * wts[hw[j] + s0 + u];
+        if (u & 1) at1[j] += v[u][j] * wts[hw[j] + i0 + u];
+        else at0[j] += v[u][j] * wts[hw[j] + i0 + u];
       }
     }
   }
@@ -299,9 +299,31 @@ __device__ __forceinline__ void merge_heads(const AttnParams &p, int kvh, int b,
     if (!ok[j]) continue;
     const int t = threadIdx.x + j * kThreads, hh = t / HD, e = t % HD;
     const float at = at0[j] + at1[j];
-    const float o = p.div_norm ? at / lsum[hh] : at * (1.0f / lsum[hh]);
-    act_st<STCOH>(p.out + static_cast<size_t>(b) * p.out_stride + (kvh * G + g0 + hh) * HD + e, o);
+    if constexpr (FINAL) {
+      const float o = p.div_norm ? at / lsum[hh] : at * (1.0f / lsum[hh]);
+      act_st<STCOH>(p.out + static_cast<size_t>(b) * p.out_stride + (kvh * G + g0 + hh) * HD + e, o);
+    } else {
+      act_st<LDCOH>(wbase + src[j], at);
+      if (e == 0) {
+        act_st<LDCOH>(wbase + src[j] - 2, mmax[hh]);
+        act_st<LDCOH>(wbase + src[j] - 1, lsum[hh]);
+      }
+    }
   }
+  __syncthreads();
+}
+
+// Counts this block in an arrival counter once every wave's stores have
+// completed; true for the last of n to arrive.  flag: LDS, free again on return.
+__device__ __forceinline__ bool last_to_arrive(unsigned *cnt, int n, int *flag) {
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (threadIdx.x == 0)
+    flag[0] = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == static_cast<unsigned>(n - 1);
+  __syncthreads();
+  const bool last = flag[0] != 0;
+  __syncthreads();
+  return last;
 }
 
 // One split block: keys [split*chunk, ...) of (stream b, kv head kvh).
@@ -358,9 +380,18 @@ __device__ __forceinline__ void attn_split_block(const AttnParams &p, int split,
   if (!appender) load_block(base0, kv0, vv0, ok0);
 
   // ---- q heads of this group (norm + rope), new k/v append ----
-  for (int g = wave; g < G; g += kWaves) {
-    const float *src = p.q + static_cast<size_t>(b) * p.q_stride + (kvh * G + g) * HD;
-    head_transform<HD, COH>(p, src, qs[g], p.q_norm_w, posi);
+  // without norm and rope a lane's q elements come straight from memory, in
+  // flight beside the first keys (no LDS round trip, no barrier)
+  const float *qsrc = p.q + static_cast<size_t>(b) * p.q_stride + kvh * G * HD;
+  const bool direct = !p.q_norm_w && !p.rope_cos;
+  float qr[G][EPL];
+  if (direct) {
+#pragma unroll
+    for (int g = 0; g < G; g++)
+#pragma unroll
+      for (int e = 0; e < EPL; e++) qr[g][e] = act_ld<COH>(qsrc, g * HD + kl * EPL + e);
+  } else {
+    for (int g = wave; g < G; g += kWaves) head_transform<HD, COH>(p, qsrc + g * HD, qs[g], p.q_norm_w, posi);
   }
   if (appender && wave == 0) {
     const float *ksrc = p.k_new + static_cast<size_t>(b) * p.kv_new_stride + kvh * HD;
@@ -373,15 +404,21 @@ __device__ __forceinline__ void attn_split_block(const AttnParams &p, int split,
       vbase[static_cast<size_t>(posi) * HD + j] = f32_to_bf16_rne(act_ld<COH>(vsrc, j));
     }
   }
-  __syncthreads();  // the appended row is read back by this block only
+  if (!direct || appender) __syncthreads();  // the appended row is read back by this block only
+  if (!direct) {
+#pragma unroll
+    for (int g = 0; g < G; g++)
+#pragma unroll
+      for (int e = 0; e < EPL; e++) qr[g][e] = qs[g][kl * EPL + e];
+  }
+  if (K8) {
+#pragma unroll
+    for (int g = 0; g < G; g++)
+#pragma unroll
+      for (int e = 0; e < EPL; e++) qr[g][e] *= p.k_scale[kvh * HD + kl * EPL + e];
+  }
 
   // ---- main loop: online softmax per lane group ----
-  float qr[G][EPL];
-#pragma unroll
-  for (int g = 0; g < G; g++)
-#pragma unroll
-    for (int e = 0; e < EPL; e++)
-      qr[g][e] = K8 ? qs[g][kl * EPL + e] * p.k_scale[kvh * HD + kl * EPL + e] : qs[g][kl * EPL + e];
   float m[G], l[G], acc[G][EPL];
 #pragma unroll
   for (int g = 0; g < G; g++) {
@@ -531,19 +568,24 @@ __device__ __forceinline__ void attn_split_block(const AttnParams &p, int split,
   }
   if constexpr (!COH) {
     if (fuse) {
-      // arrival: this wave's partial stores have completed before the count
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-      unsigned *cnt = p.cnt + static_cast<size_t>(b) * p.hkv + kvh;
+      constexpr int NE = (G * HD + kThreads - 1) / kThreads;
+      unsigned *cnt = p.cnt + (static_cast<size_t>(b) * p.hkv + kvh) * kCntWords;
       int *flag = reinterpret_cast<int *>(lds);
-      if (threadIdx.x == 0)
-        flag[0] = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                  static_cast<unsigned>(nsplits - 1);
-      __syncthreads();
-      const bool last = flag[0] != 0;
-      __syncthreads();  // the flag is read before merge_heads reuses the LDS
-      if (last) {
-        merge_heads<HD, G, (G * HD + kThreads - 1) / kThreads, true, false>(p, kvh, b, nsplits, 0, G, lds);
+      const int gs = group_size(nsplits), groups = (nsplits + gs - 1) / gs, grp = split / gs;
+      int n = nsplits, step = 1;
+      bool last = true;
+      if (groups > 1) {  // the group's last block merges the group, the last group's the groups
+        const int in_grp = min(gs, nsplits - grp * gs);
+        last = last_to_arrive(cnt + 1 + grp, in_grp, flag);
+        if (last) {
+          merge_heads<HD, G, NE, true, false, false>(p, kvh, b, grp * gs, 1, in_grp, 0, G, lds);
+          if (threadIdx.x == 0) __hip_atomic_store(cnt + 1 + grp, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        n = groups;
+        step = gs;
+      }
+      if (last && last_to_arrive(cnt, n, flag)) {
+        merge_heads<HD, G, NE, true, false, true>(p, kvh, b, 0, step, n, 0, G, lds);
         if (threadIdx.x == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
@@ -563,8 +605,14 @@ __device__ __forceinline__ void attn_merge_block(const AttnParams &p, int blk, i
   if (nsplits == 1) return;  // the split block wrote the output
   const int g0 = blk * HPB;
   if (g0 >= G) return;
-  merge_heads<HD, G, 1, COH, COH>(p, kvh, b, nsplits, g0, min(HPB, G - g0), lds);
-  __syncthreads();  // LDS is reused by the caller's next block
+  const int ng = min(HPB, G - g0), gs = group_size(nsplits), groups = (nsplits + gs - 1) / gs;
+  if (groups > 1) {
+    for (int grp = 0; grp < groups; grp++)
+      merge_heads<HD, G, 1, COH, COH, false>(p, kvh, b, grp * gs, 1, min(gs, nsplits - grp * gs), g0, ng, lds);
+    merge_heads<HD, G, 1, COH, COH, true>(p, kvh, b, 0, gs, groups, g0, ng, lds);
+  } else {
+    merge_heads<HD, G, 1, COH, COH, true>(p, kvh, b, 0, 1, nsplits, g0, ng, lds);
+  }
 }
 
 AttnParams to_params(const AttnLaunch &L);

@@ -267,8 +267,8 @@ struct AttnLaunch {
   int out_stride = 0;
   // workspace for the split partials
   float *work = nullptr;
-  // arrival counters [batch * hkv], zero between launches: the split kernel
-  // merges its partials in place (no merge launch); null: a merge follows
+  // arrival counters (attn_cnt_words()), zero between launches: the split
+  // kernel merges its partials in place (no merge launch); null: a merge follows
   unsigned *cnt = nullptr;
   int max_splits = 0;
   // int8 K / V instead of bf16 (kc / vc then hold int8 [batch, hkv, max_ctx,
@@ -278,6 +278,7 @@ struct AttnLaunch {
 };
 
 size_t attn_work_floats(int batch, int hq, int hd, int max_splits);
+size_t attn_cnt_words(int batch, int hkv);
 // Device address (resolved once per device) and capacity in floats of the
 // static split-partial workspace used by xe_attn_decode_dev_static.
 void *attn_static_scratch(int ordinal);

@@ -375,7 +375,7 @@ struct xe_decoder {
   float *arg_v = nullptr;
   int *arg_i = nullptr;
   float *attn_work = nullptr;
-  unsigned *attn_cnt = nullptr;  // split-attention arrival counters [max_batch * hkv] (self-resetting)
+  unsigned *attn_cnt = nullptr;  // split-attention arrival counters (self-resetting)
   int attn_splits = 1;
   int32_t *host_tok = nullptr;  // pinned staging [max_ctx + 1][max_batch] x 2
   int last_exec = XE_EXEC_GRAPH;  // executor of the last step launched (status messages)
@@ -634,7 +634,7 @@ void alloc_decoder(xe_decoder *d) {
   d->attn_splits = attn_splits_for(d, B, hkv_max);
   d->attn_work = dalloc<float>(attn_work_floats(static_cast<int>(part_rows), std::max(c.n_heads, 1), c.head_dim, 1),
                                s, false);
-  d->attn_cnt = dalloc<unsigned>(static_cast<size_t>(B) * hkv_max, s);  // zeroed
+  d->attn_cnt = dalloc<unsigned>(attn_cnt_words(B, hkv_max), s);  // zeroed
   if (gem) {
     const int half = c.head_dim / 2;
     std::vector<float> cs(static_cast<size_t>(c.max_ctx) * half), sn(cs.size());

@@ -98,10 +98,10 @@ void xe_ctx::ensure_attn(size_t work_floats, size_t cnt_words) {
   }
 }
 
-// Layout: [0, 256) partial maxima (w8a8_partial_floats() <= 64 floats),
-// [256, 512) scale_a, then the int8 activations.
+// Layout: [0, 1024) partial maxima (w8a8_partial_floats() <= 256 floats),
+// [1024, 1280) scale_a, then the int8 activations.
 char *xe_ctx::ensure_w8a8(size_t aq_bytes) {
-  const size_t n = 512 + aq_bytes;
+  const size_t n = 1280 + aq_bytes;
   if (n > w8a8_ws_size) {
     if (w8a8_ws) XE_HIP(hipFree(w8a8_ws));
     w8a8_ws = nullptr;
@@ -287,8 +287,8 @@ void run_w8a8(xe_ctx *ctx, const xe_weight *w, const float *x_dev, int batch, in
   const size_t n = static_cast<size_t>(batch) * w->k;
   char *ws = ctx->ensure_w8a8(n);
   float *partial = reinterpret_cast<float *>(ws);
-  float *sa = scale_a_dev ? scale_a_dev : reinterpret_cast<float *>(ws + 256);
-  int8_t *aq = reinterpret_cast<int8_t *>(ws + 512);
+  float *sa = scale_a_dev ? scale_a_dev : reinterpret_cast<float *>(ws + 1024);
+  int8_t *aq = reinterpret_cast<int8_t *>(ws + 1280);
   launch_w8a8_quant(x_dev, n, partial, aq, sa, s);
   ctx->dispatches += 2;
   W8a8Epi e;

@@ -206,20 +206,24 @@ __device__ __forceinline__ float fast_sigmoid(float x) {
   return e / (1.0f + e);
 }
 
+// The dequantised output of accumulator a: sa the activation scale, ws and
+// bias of its weight row.
+__device__ __forceinline__ float w8a8_value(int epi, int32_t a, float sa, float ws, float bias) {
+  const float v = static_cast<float>(a) * sa * ws;
+  if (epi == EPI_BIAS) return v + bias;
+  if (epi == EPI_SILU_BIAS) {
+    const float z = v + bias;
+    return z * fast_sigmoid(z);
+  }
+  return v;
+}
+
 __device__ __forceinline__ void w8a8_store(const W8a8Epi &e, int b, int r, int m, int32_t a) {
   const size_t o = static_cast<size_t>(b) * m + r;
-  if (e.acc) {
+  if (e.acc)
     e.acc[o] = a;
-    return;
-  }
-  float v = static_cast<float>(a) * e.scale_a[0] * e.ws[r];
-  if (e.epi == EPI_BIAS) {
-    v = v + e.bias[r];
-  } else if (e.epi == EPI_SILU_BIAS) {
-    const float z = v + e.bias[r];
-    v = z * fast_sigmoid(z);
-  }
-  e.y[o] = v;
+  else
+    e.y[o] = w8a8_value(e.epi, a, e.scale_a[0], e.ws[r], e.epi != EPI_NONE ? e.bias[r] : 0.0f);
 }
 
 // int8 activations x int8 weights -> int32 (exact), with the output stage

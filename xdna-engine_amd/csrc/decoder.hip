@@ -1811,13 +1811,13 @@ struct PromptWs {
   bool wide;  // every linear suits the plane kernels (wide.hip)
 };
 
-PromptWs prompt_ws(xe_decoder *d, int rows) {
+// False where the device has no room for it.
+bool prompt_ws(xe_decoder *d, int rows, PromptWs &w) {
   const auto &c = d->c;
   const size_t D = c.d_model, hq = static_cast<size_t>(c.n_heads) * c.head_dim, R = rows;
   const int kmax = static_cast<int>(std::max(std::max(D, hq), static_cast<size_t>(c.ffn)));
   // row planes (wide.hip), or the normalised rows of gemm.hip
   const size_t plane = std::max(wide_rows_floats(c.wdtype, rows, kmax), R * kmax);
-  PromptWs w{};
   size_t off = 0;
   auto take = [&](size_t floats) {
     const size_t at = off;
@@ -1832,7 +1832,13 @@ PromptWs prompt_ws(xe_decoder *d, int rows) {
     if (d->prompt_ws) XE_HIP(hipFree(d->prompt_ws));
     d->prompt_ws = nullptr;
     d->prompt_ws_bytes = 0;
-    XE_HIP(hipMalloc(reinterpret_cast<void **>(&d->prompt_ws), off));
+    const hipError_t e = hipMalloc(reinterpret_cast<void **>(&d->prompt_ws), off);
+    if (e == hipErrorOutOfMemory) {
+      d->prompt_ws = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+    XE_HIP(e);
     d->prompt_ws_bytes = off;
   }
   char *b = d->prompt_ws;
@@ -1841,7 +1847,7 @@ PromptWs prompt_ws(xe_decoder *d, int rows) {
   w.qx = at(o_qx), w.rows = at(o_rows), w.part = at(o_part), w.cnt = reinterpret_cast<unsigned *>(at(o_cnt));
   w.wide = wide_takes(std::max(std::max(static_cast<int>(d->nqkv()), c.d_model), 2 * c.ffn), kmax, rows, c.wdtype, b, 0);
   w.tok = reinterpret_cast<int32_t *>(at(o_tok)), w.pos = reinterpret_cast<int32_t *>(at(o_pos));
-  return w;
+  return true;
 }
 
 // A sublayer output on its way into the residual: a buffer, or the K splits
@@ -2043,10 +2049,13 @@ bool prompt_in_passes(xe_decoder *d, int batch, int n_prompt) {
   return (n_prompt >= 3 || (n_prompt == 2 && batch >= 2)) && batch <= kPromptRows && prompt_attn_takes(c.head_dim, c.n_heads / c.n_kv_heads);
 }
 
-// The prompt in passes over up to kPromptRows rows; h: pinned staging.
-void feed_passes(xe_decoder *d, const int32_t *prompt, int n_prompt, int batch, int32_t *h) {
+// The prompt in passes over up to kPromptRows rows; h: pinned staging.  False,
+// and nothing done, without memory for a pass.
+bool feed_passes(xe_decoder *d, const int32_t *prompt, int n_prompt, int batch, int32_t *h) {
   const int tc = std::max(1, std::min(n_prompt, kPromptRows / batch));
-  const PromptWs w = prompt_ws(d, batch * tc);
+  PromptWs w{};
+  if (!prompt_ws(d, batch * tc, w)) return false;
+  XE_HIP(hipMemsetAsync(d->stop_dev + 1, 0, batch * 4, d->s));  // no stream has stopped
   XE_HIP(hipMemsetAsync(w.cnt, 0, gemm_cnt_words() * sizeof(unsigned), d->s));
   size_t at = 0;
   for (int t0 = 0; t0 < n_prompt; t0 += tc) {
@@ -2073,6 +2082,7 @@ void feed_passes(xe_decoder *d, const int32_t *prompt, int n_prompt, int batch, 
   }
   for (const auto &ph : it->second.phases) launch_phase(ph, d->s);
   XE_HIP(hipStreamSynchronize(d->s));
+  return true;
 }
 
 // After a run of low-latency launches: a wait that timed out (or a plan the
@@ -2693,9 +2703,7 @@ void feed(xe_decoder *d, const int32_t *prompt, int n_prompt, int batch) {
   int32_t *h = d->host_tok;
   XE_REQUIRE(static_cast<size_t>(n_prompt + 1) * batch <= static_cast<size_t>(2) * (d->c.max_ctx + 2) * d->max_batch,
              "prompt too long for staging");
-  if (prompt_in_passes(d, batch, n_prompt)) {
-    XE_HIP(hipMemsetAsync(d->stop_dev + 1, 0, batch * 4, d->s));  // no stream has stopped
-    feed_passes(d, prompt, n_prompt, batch, h);
+  if (prompt_in_passes(d, batch, n_prompt) && feed_passes(d, prompt, n_prompt, batch, h)) {
     for (int b = 0; b < batch; b++) d->hpos[b] = n_prompt;
     d->live = batch;
     return;

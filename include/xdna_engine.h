@@ -246,8 +246,8 @@ int xe_attn_decode_dev(xe_ctx *ctx, const float *q_dev, const uint16_t *kc_dev,
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
  * split partials go to a static per-GPU workspace of 4 Mi floats (16 MB)
  * instead of the ctx's own; a call needing more (batch * hq * splits *
- * (hd + 2) floats, splits <= 64) fails with -1.  Same kernels and results
- * as xe_attn_decode_dev.  Calls that overlap on one GPU (any ctx, any
+ * (hd + 2) floats, splits <= 64, or up to 256 while batch * hkv * splits <=
+ * 512) fails with -1.  Same results as xe_attn_decode_dev.  Calls that overlap on one GPU (any ctx, any
  * thread) share the workspace and race: serialise them. */
 int xe_attn_decode_dev_static(xe_ctx *ctx, const float *q_dev,
                               const uint16_t *kc_dev, const uint16_t *vc_dev,

@@ -28,6 +28,7 @@ def test_grouped_merge(gpu, monkeypatch, hq, hkv, hd, ctxlen, b):
     kc = O.bf16_bits(rng.standard_normal((b, hkv, ctxlen, hd)).astype(np.float32))
     vc = O.bf16_bits(rng.standard_normal((b, hkv, ctxlen, hd)).astype(np.float32))
     scale = 1.0 / math.sqrt(hd)
+    monkeypatch.setenv("XE_ATTN_MERGE", "block")
     first = ctx.attn(q, kc, vc, lens, scale)
     again = ctx.attn(q, kc, vc, lens, scale)  # the arrival counters are zero again
     monkeypatch.setenv("XE_ATTN_MERGE", "launch")

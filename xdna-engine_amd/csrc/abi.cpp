@@ -5,6 +5,7 @@
 // Every entry point runs its body inside guard(): C++ exceptions and HIP
 // errors become a NULL / -1 return plus a thread-local message, the
 // convention of xrt_shim.cpp:42-56 and npu-capi/src/lib.rs:11-41.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -845,7 +846,10 @@ int xe_w8a8_linear(xe_ctx *ctx, const xe_weight *w, const float *x, int batch, f
 }
 
 // Splits per (stream, kv head): about XE_ATTN_WG_PER_CU (default 2)
-// workgroups per CU in total, at most one per 64 cache rows and at most 256.
+// workgroups per CU in total, at most one per 64 cache rows and at most 64, or
+// 256 while the total stays within 2 a CU (so a few streams fill the chip, and
+// the partials beyond 64 splits fit the static workspace: at most 512 x 8
+// heads x 258 floats).
 // With the merge inside the split kernel, 2 a CU against 4 (graph replays,
 // config 3): GQA 4q/1kv x 256 b = 64 ctx 4096 52.3 / 58.3 us, b = 16 ctx
 // 4096 33.0 / 47.1, b = 64 ctx 1024 26.2 / 37.2; ctx 32768 within 4 %.
@@ -859,18 +863,26 @@ static int attn_splits(const xe_ctx *ctx, int batch, int hkv, int max_ctx) {
   const int cap = (max_ctx + 63) / 64;
   ms = ms < 1 ? 1 : ms;
   ms = ms > cap ? cap : ms;
-  return ms > 256 ? 256 : ms;
+  const int top = std::min(256, std::max(64, 512 / (batch * hkv)));
+  return ms > top ? top : ms;
 }
 
 // work: the split partials (attn_work_floats(batch, hq, hd, splits) floats);
 // null = the ctx's own workspace, grown on demand, with the ctx's arrival
-// counters: the split kernel merges in place (the last split block of a
+// counters where the split kernel merges in place (the last split block of a
 // (stream, kv head) to arrive merges its partials, one launch).  A caller's
 // workspace (the allocation-free entry point) takes the separate merge launch.
-// XE_ATTN_MERGE=launch selects the merge launch for the ctx workspace too.
-static bool attn_merge_in_place() {
+// In place up to 512 outputs a (stream, kv head): its one block has all of
+// them to merge, past the L2; a launch gives every 256 outputs a block of up
+// to 1024 threads and plain loads.  us in place / launched: 4 heads x 256 of
+// one key head, one stream, 32768 keys 25.3 / 20.4, 4096 keys 15.6 / 13.2, 8
+// streams at 4096 19.0 / 16.8, 64 at 4096 52 / 50.5; 8 x 128 of two key heads,
+// two streams at 9000 keys 16.7 / 18.0; 12 x 64 at 4096 keys 8.7 / 11.9.
+// XE_ATTN_MERGE=launch or =block selects one for the ctx workspace.
+static bool attn_merge_in_place(int outs) {
   const char *e = std::getenv("XE_ATTN_MERGE");
-  return !(e && std::string(e) == "launch");
+  if (e && std::string(e) == "launch") return false;
+  return (e && std::string(e) == "block") || outs <= 512;
 }
 
 static int attn_impl(xe_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t *vc,
@@ -893,7 +905,7 @@ static int attn_impl(xe_ctx *ctx, const float *q, const uint16_t *kc, const uint
   if (work) {
     a.work = work;
   } else {
-    const bool in_place = attn_merge_in_place();
+    const bool in_place = attn_merge_in_place(hq / hkv * hd);
     ctx->ensure_attn(attn_work_floats(batch, hq, hd, a.max_splits),
                      in_place ? attn_cnt_words(batch, hkv) : 0);
     a.work = ctx->attn_work;
@@ -1095,7 +1107,7 @@ int xe_probe_attn(xe_ctx *ctx, const float *q_dev, const uint16_t *kc_dev, const
     XE_REQUIRE(batch > 0 && hq > 0 && hkv > 0 && hd > 0 && reps > 0, "bad shape");
     DeviceGuard dg(ctx->dev->ordinal);
     ctx->ensure_attn(attn_work_floats(batch, hq, hd, attn_splits(ctx, batch, hkv, max_ctx)),
-                     attn_merge_in_place() ? attn_cnt_words(batch, hkv) : 0);  // no allocation under capture
+                     attn_merge_in_place(hq / hkv * hd) ? attn_cnt_words(batch, hkv) : 0);  // no allocation under capture
     *us_per_call = time_captured(ctx, reps, flags, [&]() {
       attn_impl(ctx, q_dev, kc_dev, vc_dev, lens_dev, batch, hq, hkv, hd, max_ctx, scale, out_dev);
     });

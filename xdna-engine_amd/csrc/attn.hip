@@ -63,6 +63,11 @@ __global__ __launch_bounds__(kThreads) void attn_merge_kernel(AttnParams p) {
   adev::attn_merge_block<HD, G, false>(p, blockIdx.x, blockIdx.y, blockIdx.z, lds);
 }
 
+template <int HD, int G>
+__global__ __launch_bounds__(adev::team_threads(HD, G) * adev::kTeams) void attn_merge_wide_kernel(AttnParams p) {
+  adev::attn_merge_wide<HD, G>(p, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
 using AttnFn = void (*)(AttnParams);
 
 template <int HD>
@@ -72,6 +77,17 @@ AttnFn pick_g(int g, bool merge, bool shared) {
     case 2: return merge ? attn_merge_kernel<HD, 2> : attn_kernel<HD, 2>;
     case 4: return merge ? attn_merge_kernel<HD, 4> : attn_kernel<HD, 4>;
     case 8: return merge ? attn_merge_kernel<HD, 8> : attn_kernel<HD, 8>;
+  }
+  return nullptr;
+}
+
+template <int HD>
+AttnFn pick_merge_wide(int g) {
+  switch (g) {
+    case 1: return attn_merge_wide_kernel<HD, 1>;
+    case 2: return attn_merge_wide_kernel<HD, 2>;
+    case 4: return attn_merge_wide_kernel<HD, 4>;
+    case 8: return attn_merge_wide_kernel<HD, 8>;
   }
   return nullptr;
 }
@@ -111,6 +127,16 @@ AttnFn pick(int hd, int g, bool merge, int kv8 = 0, bool shared = false) {
 
 int kv8_of(const AttnParams &p) { return (p.k_scale ? 1 : 0) | (p.v_scale ? 2 : 0); }
 
+// The merge after a split launch without arrival counters: beyond one group
+// of splits the merge in groups, up to 1024 threads a block.
+void launch_merge(const AttnParams &p, int hd, int g, hipStream_t s) {
+  const int blocks = (g * hd + kThreads - 1) / kThreads;
+  const bool wide = p.max_splits > adev::kGroup;
+  const AttnFn fn = !wide ? pick(hd, g, true) : hd == 64 ? pick_merge_wide<64>(g) : hd == 128 ? pick_merge_wide<128>(g) : pick_merge_wide<256>(g);
+  hipLaunchKernelGGL(fn, dim3(blocks, p.hkv, p.batch), dim3(wide ? adev::team_threads(hd, g) * adev::kTeams : kThreads), 0, s, p);
+  XE_HIP(hipGetLastError());
+}
+
 }  // namespace
 
 // One attention phase of a step: split partials or the merge (none with
@@ -122,12 +148,11 @@ void launch_attn_phase(const sdev::Phase &ph, hipStream_t s) {
   AttnFn fn = pick(ph.hd, ph.g, merge, kv8_of(p), p.kv_bstride == 0 && p.batch > 1);
   XE_REQUIRE(fn, "attn phase: unsupported head_dim / group (int8 K/V: one query head a KV head)");
   if (merge) {
-    const int blocks = (ph.g * ph.hd + kThreads - 1) / kThreads;
-    hipLaunchKernelGGL(fn, dim3(blocks, p.hkv, p.batch), dim3(kThreads), 0, s, p);
+    launch_merge(p, ph.hd, ph.g, s);
   } else {
     hipLaunchKernelGGL(fn, dim3(p.max_splits, p.hkv, p.batch), dim3(kThreads), 0, s, p);
+    XE_HIP(hipGetLastError());
   }
-  XE_HIP(hipGetLastError());
 }
 
 size_t attn_cnt_words(int batch, int hkv) { return static_cast<size_t>(batch) * hkv * adev::kCntWords; }
@@ -183,11 +208,7 @@ void launch_attn(const AttnLaunch &L, hipStream_t s) {
   XE_REQUIRE(!kv8_of(p) || !L.k_new, "attn: int8 K/V caches take no append");
   hipLaunchKernelGGL(fn, dim3(L.max_splits, L.hkv, L.batch), dim3(kThreads), 0, s, p);
   XE_HIP(hipGetLastError());
-  if (L.max_splits > 1 && !L.cnt) {
-    const int blocks = (g * L.hd + kThreads - 1) / kThreads;
-    hipLaunchKernelGGL(merge, dim3(blocks, L.hkv, L.batch), dim3(kThreads), 0, s, p);
-    XE_HIP(hipGetLastError());
-  }
+  if (L.max_splits > 1 && !L.cnt) launch_merge(p, L.hd, g, s);
 }
 
 }  // namespace xe

@@ -53,7 +53,8 @@ constexpr int kMaxSplits = 256;
 // block reads at most kGroup partials, so a long context of few streams can
 // split over the whole chip.  4 heads x 256, one key head, us, all splits (64
 // at most) merged by one block / in groups: 32768 keys of one stream 47.4 /
-// 25.5 (256 splits), 4096 keys of one 29.3 / 16.0, of 8 streams 32.6 / 19.5.
+// 25.5 (256 splits), 4096 keys of one 29.3 / 16.0, of 8 streams 32.6 / 19.5
+// (merged in the split kernel; attn_merge_wide is faster still at this size).
 constexpr int kGroup = 16;  // partials a merge takes, and groups
 static_assert(kGroup * kGroup >= kMaxSplits, "two levels of groups cover every split count");
 constexpr int kCntWords = 1 + kGroup;  // arrival counters of a (stream, kv head)
@@ -593,8 +594,8 @@ __device__ __forceinline__ void attn_split_block(const AttnParams &p, int split,
   __syncthreads();  // LDS is reused by the caller's next block
 }
 
-// Merge block `blk` of (stream b, kv head kvh): outputs blk*256 .. +256 of the
-// G*HD, i.e. heads [blk * HPB, +HPB) with HPB = 256 / HD.
+// Merge block `blk` of (stream b, kv head kvh), at most kGroup splits: outputs
+// blk*256 .. +256 of the G*HD, i.e. heads [blk * HPB, +HPB) with HPB = 256 / HD.
 template <int HD, int G, bool COH>
 __device__ __forceinline__ void attn_merge_block(const AttnParams &p, int blk, int kvh, int b, float *lds) {
   constexpr int HPB = kThreads >= HD ? kThreads / HD : 1;  // heads per block
@@ -605,14 +606,100 @@ __device__ __forceinline__ void attn_merge_block(const AttnParams &p, int blk, i
   if (nsplits == 1) return;  // the split block wrote the output
   const int g0 = blk * HPB;
   if (g0 >= G) return;
+  merge_heads<HD, G, 1, COH, COH, true>(p, kvh, b, 0, 1, nsplits, g0, min(HPB, G - g0), lds);
+}
+
+// The same for any split count, in groups: the block's outputs (at most 256)
+// are taken by kTeams teams of a thread each, team t the groups t, t + kTeams,
+// ..., and the groups merge through LDS.  The same sums in the same order as the split
+// kernel's own merge.  Every partial a thread takes is loaded before the
+// weights, so the merge is one memory round trip whatever the split count.
+// 4 heads x 256 of one key head, one stream, split and merge, us: 32768 keys
+// 34.9 (256 threads, one level, at most 64 splits) -> 20.3, 4096 keys 16.6 ->
+// 13.1, 8 streams at 4096 keys 20.4 -> 16.8.
+constexpr int kTeams = 4;
+__host__ __device__ constexpr int team_threads(int hd, int g) { return g * hd < kThreads ? g * hd : kThreads; }
+template <int HD, int G>
+__device__ __forceinline__ void attn_merge_wide(const AttnParams &p, int blk, int kvh, int b) {
+  constexpr int RS = HD + 2;
+  constexpr int HPB = kThreads >= HD ? kThreads / HD : 1;
+  constexpr int NG = kGroup / kTeams;  // groups a team takes
+  constexpr int TT = team_threads(HD, G), TW = TT / 64;
+  __shared__ float wts[HPB][kGroup][kGroup], gw[HPB][kGroup], lsum[HPB][kGroup], mmax[HPB][kGroup], fsum[HPB];
+  __shared__ float gacc[kGroup][TT];
+  const int len = stream_len(p, b);
+  if (len <= 0) return;
+  int chunk, nsplits;
+  split_range(len, p.max_splits, chunk, nsplits);
+  if (nsplits == 1) return;  // the split block wrote the output
+  const int g0 = blk * HPB;
+  if (g0 >= G) return;
   const int ng = min(HPB, G - g0), gs = group_size(nsplits), groups = (nsplits + gs - 1) / gs;
-  if (groups > 1) {
-    for (int grp = 0; grp < groups; grp++)
-      merge_heads<HD, G, 1, COH, COH, false>(p, kvh, b, grp * gs, 1, min(gs, nsplits - grp * gs), g0, ng, lds);
-    merge_heads<HD, G, 1, COH, COH, true>(p, kvh, b, 0, gs, groups, g0, ng, lds);
-  } else {
-    merge_heads<HD, G, 1, COH, COH, true>(p, kvh, b, 0, 1, nsplits, g0, ng, lds);
+  const float *wbase = p.work + (static_cast<size_t>(b) * p.hq + kvh * G + g0) * p.max_splits * RS;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int team = wave / TW, t = threadIdx.x % TT;
+  const bool ok = t < ng * HD;
+  const int hh = ok ? t / HD : 0, e = t % HD;
+  float v[NG][kGroup];
+#pragma unroll
+  for (int j = 0; j < NG; j++) {
+    const int s0 = (team + j * kTeams) * gs;
+#pragma unroll
+    for (int i = 0; i < kGroup; i++)
+      if (i < gs && s0 + i < nsplits) v[j][i] = wbase[(hh * p.max_splits + s0 + i) * RS + 2 + e];
   }
+  // a wave an (group, head): the partials' weights, as merge_weights does
+  for (int id = wave; id < groups * ng; id += kTeams * TW) {
+    const int grp = id % groups, h = id / groups, n = min(gs, nsplits - grp * gs);
+    const bool on = lane < n;
+    const int src = (h * p.max_splits + grp * gs + (on ? lane : 0)) * RS;
+    const float ms = wbase[src], lv = wbase[src + 1];
+    float mx = on ? ms : -INFINITY;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    const float f = !on || ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
+    if (on) wts[h][grp][lane] = f;
+    const float ls = wave_sum(on ? lv * f : 0.f);
+    if (lane == 0) {
+      lsum[h][grp] = ls;
+      mmax[h][grp] = mx;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NG; j++) {
+    const int grp = team + j * kTeams;
+    if (grp >= groups) continue;
+    float at0 = 0.f, at1 = 0.f;
+#pragma unroll
+    for (int i = 0; i < kGroup; i++) {
+      if (i >= gs || grp * gs + i >= nsplits) continue;
+      if (i & 1) at1 += v[j][i] * wts[hh][grp][i];
+      else at0 += v[j][i] * wts[hh][grp][i];
+    }
+    gacc[grp][t] = at0 + at1;
+  }
+  if (wave < ng) {  // the groups' weights
+    const bool on = lane < groups;
+    const float ms = mmax[wave][on ? lane : 0], lv = lsum[wave][on ? lane : 0];
+    float mx = on ? ms : -INFINITY;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    const float f = !on || ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
+    if (on) gw[wave][lane] = f;
+    const float ls = wave_sum(on ? lv * f : 0.f);
+    if (lane == 0) fsum[wave] = groups > 1 ? ls : lv;
+  }
+  __syncthreads();
+  if (team != 0 || !ok) return;
+  float at0 = 0.f, at1 = 0.f;
+  for (int i = 0; i < groups; i++) {
+    if (i & 1) at1 += gacc[i][t] * gw[hh][i];
+    else at0 += gacc[i][t] * gw[hh][i];
+  }
+  const float at = groups > 1 ? at0 + at1 : gacc[0][t];
+  p.out[static_cast<size_t>(b) * p.out_stride + (kvh * G + g0 + hh) * HD + e] =
+      p.div_norm ? at / fsum[hh] : at * (1.0f / fsum[hh]);
 }
 
 AttnParams to_params(const AttnLaunch &L);

@@ -875,9 +875,10 @@ static int attn_splits(const xe_ctx *ctx, int batch, int hkv, int max_ctx) {
 // In place up to 512 outputs a (stream, kv head): its one block has all of
 // them to merge, past the L2; a launch gives every 256 outputs a block of up
 // to 1024 threads and plain loads.  us in place / launched: 4 heads x 256 of
-// one key head, one stream, 32768 keys 25.3 / 20.4, 4096 keys 15.6 / 13.2, 8
-// streams at 4096 19.0 / 16.8, 64 at 4096 52 / 50.5; 8 x 128 of two key heads,
-// two streams at 9000 keys 16.7 / 18.0; 12 x 64 at 4096 keys 8.7 / 11.9.
+// one key head, one stream, 32768 keys 25.3 / 17.7, 4096 keys 15.6 / 11.7, 8
+// streams at 4096 19.0 / 15.3, 64 at 4096 52 / 50.3; 8 x 128 of two key heads,
+// two streams at 9000 keys 16.8 / 15.1 (the line lies above it: one size only);
+// 12 x 64, two streams at 4096 keys 9.1 / 10.0, one at 448 6.6 / 7.7.
 // XE_ATTN_MERGE=launch or =block selects one for the ctx workspace.
 static bool attn_merge_in_place(int outs) {
   const char *e = std::getenv("XE_ATTN_MERGE");

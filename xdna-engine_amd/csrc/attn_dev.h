@@ -615,8 +615,9 @@ __device__ __forceinline__ void attn_merge_block(const AttnParams &p, int blk, i
 // kernel's own merge.  Every partial a thread takes is loaded before the
 // weights, so the merge is one memory round trip whatever the split count.
 // 4 heads x 256 of one key head, one stream, split and merge, us: 32768 keys
-// 34.9 (256 threads, one level, at most 64 splits) -> 20.3, 4096 keys 16.6 ->
-// 13.1, 8 streams at 4096 keys 20.4 -> 16.8.
+// 34.9 (256 threads, one level, at most 64 splits) -> 17.7, 4096 keys 16.6 ->
+// 11.7, 8 streams at 4096 keys 20.4 -> 15.3 (20.3 / 13.1 / 16.8 with a branch
+// a load instead of clamped loads at weight zero).
 constexpr int kTeams = 4;
 __host__ __device__ constexpr int team_threads(int hd, int g) { return g * hd < kThreads ? g * hd : kThreads; }
 template <int HD, int G>
@@ -644,9 +645,14 @@ __device__ __forceinline__ void attn_merge_wide(const AttnParams &p, int blk, in
 #pragma unroll
   for (int j = 0; j < NG; j++) {
     const int s0 = (team + j * kTeams) * gs;
+    if (s0 >= nsplits) continue;
+    // past the last split: that one again, with weight zero
+    auto ld = [&](int i) { v[j][i] = wbase[(hh * p.max_splits + min(s0 + i, nsplits - 1)) * RS + 2 + e]; };
 #pragma unroll
-    for (int i = 0; i < kGroup; i++)
-      if (i < gs && s0 + i < nsplits) v[j][i] = wbase[(hh * p.max_splits + s0 + i) * RS + 2 + e];
+    for (int i = 0; i < kGroup / 2; i++) ld(i);
+    if (gs == kGroup)
+#pragma unroll
+      for (int i = kGroup / 2; i < kGroup; i++) ld(i);
   }
   // a wave an (group, head): the partials' weights, as merge_weights does
   for (int id = wave; id < groups * ng; id += kTeams * TW) {
@@ -658,7 +664,7 @@ __device__ __forceinline__ void attn_merge_wide(const AttnParams &p, int blk, in
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
     const float f = !on || ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mx);
-    if (on) wts[h][grp][lane] = f;
+    if (lane < kGroup) wts[h][grp][lane] = f;
     const float ls = wave_sum(on ? lv * f : 0.f);
     if (lane == 0) {
       lsum[h][grp] = ls;
@@ -671,12 +677,15 @@ __device__ __forceinline__ void attn_merge_wide(const AttnParams &p, int blk, in
     const int grp = team + j * kTeams;
     if (grp >= groups) continue;
     float at0 = 0.f, at1 = 0.f;
-#pragma unroll
-    for (int i = 0; i < kGroup; i++) {
-      if (i >= gs || grp * gs + i >= nsplits) continue;
+    auto add = [&](int i) {
       if (i & 1) at1 += v[j][i] * wts[hh][grp][i];
       else at0 += v[j][i] * wts[hh][grp][i];
-    }
+    };
+#pragma unroll
+    for (int i = 0; i < kGroup / 2; i++) add(i);
+    if (gs == kGroup)
+#pragma unroll
+      for (int i = kGroup / 2; i < kGroup; i++) add(i);
     gacc[grp][t] = at0 + at1;
   }
   if (wave < ng) {  // the groups' weights

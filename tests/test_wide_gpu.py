@@ -88,3 +88,49 @@ def test_prompt_passes_logits(gpu, xe, family, wd, batch, n):
     compare_logits(got, want, "prompt-%s-%s-b%d-n%d" % (family, wd, batch, n))
     dec.close()
     om.close()
+
+
+@pytest.mark.parametrize("wd", ["i8", "i4"])
+@pytest.mark.parametrize("m,k,b", [(4100, 4096, 509), (4590, 640, 475)])
+def test_wide_linear_range_within_a_row(gpu, xe, wd, m, k, b):
+    """Rows whose elements differ by up to the whole fp32 range: one large
+    element under a zero weight column, magnitudes spread over 2^-100 .. 2^100
+    under weights that are non-zero in 48 columns only, between ordinary rows
+    and in tiles of ordinary rows.  Bars: dense rows as above (they sum K
+    comparable products); an output of n = 48 products within (n + 8) 2^-24 of
+    the sum of their magnitudes (n roundings of an fp32 sum, operands to
+    2^-23 each, the scale)."""
+    _, ctx = gpu
+    print("[case] wide range %s m=%d k=%d b=%d" % (wd, m, k, b), flush=True)
+    rng = np.random.default_rng(m + b)
+    x = rng.standard_normal((b, k)).astype(np.float32)
+    few = np.sort(rng.choice(np.arange(8, k), 48, replace=False))
+    w = rng.standard_normal((m, k)).astype(np.float32)
+    w[:, :8] = 0.0
+    w[-64:] = 0.0
+    w[-64:, few] = rng.standard_normal((64, 48)).astype(np.float32)
+    ratios = [2.0 ** e for e in (8, 16, 20, 24, 26, 27, 28, 29, 30, 31, 36, 43, 60, 100)] + [1e9, 1e13, 1e30]
+    at = rng.permutation(130)[:len(ratios)].tolist() + list(range(b - len(ratios), b))
+    for r, ratio in zip(at, ratios * 2):
+        x[r, r % 8] = ratio
+    for r in (130, 131, b - 20):
+        x[r] *= np.exp2(rng.integers(-100, 101, k)).astype(np.float32)
+    x[132] = 0.0
+    x[133] *= np.float32(2.0 ** -120)  # a small row: nothing is out of its range
+    x[134, few[:24]] *= np.float32(2.0 ** -90)
+    if wd == "i8":
+        q, s = O.quant_rows_i8(w)
+        h, val = ctx.register_weight_q8(q, s), q.astype(np.float64) * s[:, None].astype(np.float64)
+    else:
+        q, s = O.quant_rows_i4(w)
+        h, val = ctx.register_weight_q4(q, s), O.unpack_i4(q).astype(np.float64) * s[:, None].astype(np.float64)
+    got = ctx.gemv(h, x)
+    h.free()
+    want = x.astype(np.float64) @ val.T
+    size = np.abs(x).astype(np.float64) @ np.abs(val).T
+    diff = np.abs(got - want)
+    few_err = (diff[:, -64:] / np.maximum(size[:, -64:], 1e-300)).max(axis=1)
+    assert few_err.max() <= 56 * 2.0 ** -24, "row %d: %g of its products" % (few_err.argmax(), few_err.max())
+    dense = np.linalg.norm(got - want, axis=1) / np.maximum(np.linalg.norm(want, axis=1), 1e-300)
+    dense[[130, 131, b - 20]] = 0.0  # of few dominant products: the bound above
+    assert dense.max() <= 2e-6, "row %d rel-L2 %g" % (dense.argmax(), dense.max())

@@ -1903,7 +1903,7 @@ void prompt_linear(xe_decoder *d, const PromptWs &w, GemvCall g, int n, const Pe
   q.m = m.rows;
   q.k = m.cols;
   q.n = n;
-  q.rows = wide_rows_in(w.rows, n);
+  q.rows = wide_rows_in(w.rows, n, m.cols);
   q.act = g.act;
   q.y = g.y;
   q.ldy = g.ldy;
@@ -2169,7 +2169,7 @@ void precompute_cross(xe_decoder *d) {
     float *p;
     ~Free() { (void)hipFree(p); }
   } fr{tmp};
-  const WideRows rows = wide_rows_in(tmp + n_tmp, T);
+  const WideRows rows = wide_rows_in(tmp + n_tmp, T, D);
   if (wide) {
     gdev::GemvParams p{};
     p.x = d->enc;

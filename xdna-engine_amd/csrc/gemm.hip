@@ -1487,7 +1487,7 @@ void launch_gemm_op(const GemvLaunch &L, float *xn, float *ws, unsigned *cnt, hi
     g.m = L.m;
     g.k = L.k;
     g.n = L.batch;
-    g.rows = wide_rows_in(xn, L.batch);
+    g.rows = wide_rows_in(xn, L.batch, L.k);
     g.y = L.y;
     g.ldy = L.ldy;
     g.ws = ws;

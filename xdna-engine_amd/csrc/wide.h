@@ -9,24 +9,31 @@ namespace xe {
 
 // Rows as planes: x = sum of 16-bit parts, plane q of row r at
 // planes[(q * n + r) * k + i].
-//   int8 / int4 weights   2 fp16 parts of x * 2^rexp[r] (rexp: the power of
-//                         two that puts the row's largest |x| in [2^14, 2^15))
+//   int8 / int4 weights   2 fp16 parts of x * 2^s (s in rexp[r]: the power of
+//                         two that puts the row's largest |x| in [2^14,
+//                         2^15)), the second one times 2^12.  Blocks of 64
+//                         elements, one of them not zero and below 2^-28 of
+//                         that: the fp32 bits, upper and lower halves (raw
+//                         says which blocks)
 //   bf16 / bfp16 weights  3 bf16 parts of x, exactly
 struct WideRows {
   uint16_t *planes = nullptr;
-  int *rexp = nullptr;  // wide_rexp_ints(n) ints (int8 / int4 weights)
+  int *rexp = nullptr;     // wide_rexp_ints(n) ints (int8 / int4 weights)
+  uint8_t *raw = nullptr;  // wide_raw_ints(n, k) ints (int8 / int4 weights)
 };
 int wide_planes(int wdtype);
 size_t wide_plane_elems(int wdtype, int n, int k);
 size_t wide_rexp_ints(int n);
-// One buffer for both: floats it takes, and the two halves of it.
+size_t wide_raw_ints(int n, int k);
+// One buffer for all three: floats it takes, and its parts.
 inline size_t wide_rows_floats(int wdtype, int n, int k) {
-  return wide_rexp_ints(n) + (wide_plane_elems(wdtype, n, k) + 1) / 2;
+  return wide_rexp_ints(n) + wide_raw_ints(n, k) + (wide_plane_elems(wdtype, n, k) + 1) / 2;
 }
-inline WideRows wide_rows_in(float *buf, int n) {
+inline WideRows wide_rows_in(float *buf, int n, int k) {
   WideRows r;
   r.rexp = reinterpret_cast<int *>(buf);
-  r.planes = reinterpret_cast<uint16_t *>(buf + wide_rexp_ints(n));
+  r.raw = reinterpret_cast<uint8_t *>(buf + wide_rexp_ints(n));
+  r.planes = reinterpret_cast<uint16_t *>(buf + wide_rexp_ints(n) + wide_raw_ints(n, k));
   return r;
 }
 

@@ -10,12 +10,15 @@
 // the few rows of a decode step and costs more than the MFMAs from about a
 // hundred rows on).
 //   int8 / int4 weights are whole numbers below 2^11, exact in fp16, so two
-//   fp16 parts do: x 2^s = hi + lo + e, |e| <= 2^-22 |x| (round to nearest
-//   each), with s per row putting the largest |x| in [2^14, 2^15), so parts
-//   keep their full 11 bits down to 2^-17 of the row's largest value and an
-//   absolute error of 2^-40 of it below that.  Two parts round like fp32
-//   itself does: the error against 64 bits is that of the fp32 sums (2.1e-7
-//   at 13824 x 1152 x 512 rows with either split).
+//   fp16 parts do: x 2^s = hi + lo 2^-12 + e, round to nearest each, with s
+//   per row putting the largest |x| in [2^14, 2^15).  The second part is kept
+//   2^12 larger and meets weights 2^12 smaller (exact as well), so |e| <=
+//   2^-23 |x 2^s| down to 2^-14, 2^-28 of the row's largest value: the last
+//   of 24 bits.  The error against 64 bits is that of the fp32 sums (2.1e-7 at
+//   13824 x 1152 x 512 rows with either split).  A block of 64 elements with a
+//   smaller one (zeros aside) is stored as its fp32 bits instead, and a GEMM
+//   tile takes the steps of its blocks like that last, all their rows split
+//   into three bf16 parts, exactly, like the kernels of gemm.hip.
 //   bf16 / bfp16 weights have an 8-bit exponent, which fp16 does not hold:
 //   three bf16 parts, x = hi + mid + lo exactly, as in gemm.hip.
 #include <algorithm>
@@ -44,6 +47,18 @@ constexpr int kMaxK = 16384;        // rows kernel: 16 float4 a thread
 constexpr int kMaxKs = 8;           // K splits
 constexpr int kRowPad = 128;        // rexp is readable up to a multiple of it
 constexpr int kLds = 160 * 1024;    // LDS of a CU
+constexpr int kLoExp = 12;          // fp16 parts: the second one is kept 2^kLoExp larger
+constexpr int kMaxSteps = kMaxK / kBK;
+
+// rexp of a row: its s, and above it whether blocks of the row are stored as
+// fp32: upper halves in plane 0, lower halves in plane 1
+__host__ __device__ __forceinline__ int rexp_word(int s, bool raw) { return (s & 0xffff) | (raw ? 1 << 16 : 0); }
+__device__ __forceinline__ int rexp_s(int w) { return static_cast<int16_t>(w); }
+__device__ __forceinline__ bool rexp_raw(int w) { return (w >> 16) & 1; }
+// byte of (row, step) in the flags behind rexp, written for rows with rexp_raw
+__device__ __forceinline__ size_t raw_at(int row, int step, int steps) {
+  return (static_cast<size_t>(row / kRowPad) * steps + step) * kRowPad + row % kRowPad;
+}
 
 template <int WT>
 constexpr int planes_of() {
@@ -56,6 +71,9 @@ constexpr int planes_of() {
 __device__ __forceinline__ uint32_t pack_hi16(float lo, float hi) {
   return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
+__device__ __forceinline__ uint32_t pack_lo16(float lo, float hi) {
+  return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x05040100u);
+}
 __device__ __forceinline__ float trunc_bf16(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
 
 __device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
@@ -64,11 +82,13 @@ __device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast
 // A thread holds float4 chunks threadIdx.x + 256 j, j < NV, from the first
 // load to the plane stores (K <= 1024 NV), so the row is read once.  Bound by
 // its chain of block reductions (one per norm statistic, one for the row's
-// largest |h|), which the other rows' workgroups of the CU overlap.
+// largest and smallest |h|), which the other rows' workgroups of the CU
+// overlap.
 template <int NV, int P>
-__global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint16_t *planes, int *rexp) {
+__global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint16_t *planes, int *rexp, uint8_t *raw_flags) {
   __shared__ float red[2 * 4 * gdev::kMaxWaves];
   __shared__ float mx[kT / 64];
+  __shared__ float mn[kT / 64];
   const int b = blockIdx.x, K = p.k, K4 = K / 4;
   const float fk = static_cast<float>(K);
   float t[NV][4], g[NV][4], be[NV][4];
@@ -179,20 +199,35 @@ __global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint1
       }
   }
   if constexpr (P == 2) {
+    // the largest |h|, and the smallest that is not zero (bits of 2 |h| less
+    // one: zero comes last)
     float a = 0.f;
+    uint32_t low = ~0u;
 #pragma unroll
     for (int j = 0; j < NV; j++)
       if (static_cast<int>(threadIdx.x) + j * kT < K4)
 #pragma unroll
-        for (int c = 0; c < 4; c++) a = fmaxf(a, fabsf(t[j][c]));
+        for (int c = 0; c < 4; c++) {
+          a = fmaxf(a, fabsf(t[j][c]));
+          low = min(low, 2u * __float_as_uint(t[j][c]) - 1u);
+        }
     a = gdev::wave_max(a);
-    if ((threadIdx.x & 63) == 0) mx[threadIdx.x >> 6] = a;
+    float least = -gdev::wave_max(low != ~0u ? -__uint_as_float((low >> 1) + 1u) : -INFINITY);
+    if ((threadIdx.x & 63) == 0) {
+      mx[threadIdx.x >> 6] = a;
+      mn[threadIdx.x >> 6] = least;
+    }
     __syncthreads();
     a = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
+    least = fminf(fminf(mn[0], mn[1]), fminf(mn[2], mn[3]));
     int e = 0;
     if (a > 0.f && a < INFINITY) (void)frexpf(a, &e);  // a in [2^(e-1), 2^e)
-    const int s = 15 - e;
-    if (threadIdx.x == 0) rexp[b] = s;
+    int s = 15 - e;
+    least = __builtin_ldexpf(least, s);
+    const bool raw = least < 0x1p-14f;
+    const bool all = least < 0x1p-85f;  // more than x 2^s holds as well: every block as x itself
+    if (all) s = 0;
+    if (threadIdx.x == 0) rexp[b] = rexp_word(s, raw);
 #pragma unroll
     for (int j = 0; j < NV; j++) {
       const int i = static_cast<int>(threadIdx.x) + j * kT;
@@ -205,7 +240,18 @@ __global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint1
       for (int c = 0; c < 4; c++) {
         const float v = __builtin_ldexpf(t[j][c], s);
         hi.h[c] = static_cast<_Float16>(v);
-        lo.h[c] = static_cast<_Float16>(v - static_cast<float>(hi.h[c]));
+        lo.h[c] = static_cast<_Float16>((v - static_cast<float>(hi.h[c])) * static_cast<float>(1 << kLoExp));
+      }
+      if (raw) {  // a block is 16 lanes
+        bool low4 = all;
+#pragma unroll
+        for (int c = 0; c < 4; c++) low4 |= t[j][c] != 0.f && fabsf(__builtin_ldexpf(t[j][c], s)) < 0x1p-14f;
+        const bool blk = ((__ballot(low4) >> (threadIdx.x & 48)) & 0xffffu) != 0;
+        if ((threadIdx.x & 15) == 0) raw_flags[raw_at(b, i / (kBK / 4), (K + kBK - 1) / kBK)] = blk;
+        if (blk) {
+          hi.u = u32x2{pack_hi16(t[j][0], t[j][1]), pack_hi16(t[j][2], t[j][3])};
+          lo.u = u32x2{pack_lo16(t[j][0], t[j][1]), pack_lo16(t[j][2], t[j][3])};
+        }
       }
       const size_t o = static_cast<size_t>(b) * K + 4 * i;
       *reinterpret_cast<u32x2 *>(planes + o) = hi.u;
@@ -241,6 +287,7 @@ struct WideParams {
   int m, k, n;
   const uint16_t *planes;
   const int *rexp;
+  const uint8_t *raw;
   int act;
   float *y;
   int ldy;
@@ -260,10 +307,11 @@ __device__ __forceinline__ float gelu_tanh_wide(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * u2));
 }
 
-// LDS offset of the epilogue's tables: behind the operand buffers and the
-// waves' output areas (which overlap).
+// LDS offset of the epilogue's tables (and of what says which steps run on
+// fp32 rows): behind the operand buffers and the waves' output areas (which
+// overlap).
 constexpr int epi_offset(int buffers, int out) { return ((buffers > out ? buffers : out) + 15) / 16 * 16; }
-constexpr int epi_tables(int bx, int bw) { return 4 * (bx + 2 * bw); }
+constexpr int epi_tables(int bx, int bw) { return 4 * (bx + 2 * bw) + 48 + 2 * kMaxSteps; }
 
 template <int WT>
 struct WTraits {
@@ -324,6 +372,31 @@ __device__ __forceinline__ bf16x8 bfp_to_bf16(uint32_t q0, uint32_t q1, uint32_t
   }
   const u32x4 o = {pack_hi16(f[0], f[1]), pack_hi16(f[2], f[3]), pack_hi16(f[4], f[5]), pack_hi16(f[6], f[7])};
   return __builtin_bit_cast(bf16x8, o);
+}
+
+// The same numbers as bf16: 8 int8, 8 int4
+__device__ __forceinline__ bf16x8 i8_to_bf16(uint32_t q0, uint32_t q1) {
+  float f[8];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    f[i] = static_cast<float>(static_cast<int>(__builtin_amdgcn_sbfe(static_cast<int>(q0), 8 * i, 8)));
+    f[4 + i] = static_cast<float>(static_cast<int>(__builtin_amdgcn_sbfe(static_cast<int>(q1), 8 * i, 8)));
+  }
+  const u32x4 o = {pack_hi16(f[0], f[1]), pack_hi16(f[2], f[3]), pack_hi16(f[4], f[5]), pack_hi16(f[6], f[7])};
+  return __builtin_bit_cast(bf16x8, o);
+}
+__device__ __forceinline__ bf16x8 i4_to_bf16(uint32_t q) {
+  float f[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) f[i] = static_cast<float>(static_cast<int>(__builtin_amdgcn_sbfe(static_cast<int>(q), 4 * i, 4)));
+  const u32x4 o = {pack_hi16(f[0], f[1]), pack_hi16(f[2], f[3]), pack_hi16(f[4], f[5]), pack_hi16(f[6], f[7])};
+  return __builtin_bit_cast(bf16x8, o);
+}
+
+// fp16 weights for the second part of the rows
+__device__ __forceinline__ u32x4 lo_weights(u32x4 w) {
+  const f16x8 v = __builtin_bit_cast(f16x8, w) * static_cast<_Float16>(1.0f / (1 << kLoExp));
+  return __builtin_bit_cast(u32x4, v);
 }
 
 template <int WT>
@@ -405,7 +478,15 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
     u32x4 w[NW];
     uint32_t e[NW];
   };
-  auto issue = [&](int step, Stage &st) {  // past the last step: zeros
+  // tables behind the operand buffers: the rows' exponents, the weight rows'
+  // scales and biases; a word a wave (fp32 blocks among its rows), the number
+  // of steps without any, the steps in the order they are taken, their flags
+  int *const rs = reinterpret_cast<int *>(lds + kEpi);
+  float *const wsc = reinterpret_cast<float *>(rs + BX), *const wbi = wsc + BW;
+  int *const seen = reinterpret_cast<int *>(wbi + BW);
+  uint8_t *const order = reinterpret_cast<uint8_t *>(seen + 12), *const hit = order + kMaxSteps;
+  int nfast = nsteps;  // steps without fp32 blocks: all in their order, or the first nfast of `order`
+  auto issue_at = [&](int step, Stage &st) {  // past the last step: zeros
     const int k0 = (step0 + step) * kBK;
     const bool xok = k0 + 8 * xc < kend, wok = k0 + KPC * wc < kend;
 #pragma unroll
@@ -424,12 +505,14 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
         st.e[j] = __builtin_amdgcn_raw_buffer_load_b16(re, wok ? eoff[j] : kNoRec, k0 / 8, 0);
     }
   };
+  auto issue = [&](int step, Stage &st, auto sorted) {
+    if constexpr (decltype(sorted)::value) step = step < nfast ? __builtin_amdgcn_readfirstlane(order[step]) : nsteps;
+    issue_at(step, st);
+  };
   const int xput = lds_chunk<128>(xr, xc);
   const int wput = WT == XE_I4 ? lds_chunk<32>(wr, wc >> 1) + 8 * (wc & 1) : lds_chunk<ROWB>(wr, wc);
-  auto put = [&](int buf, const Stage &st) {
-    uint8_t *xs = lds + buf, *ws = xs + XB, *es = ws + WB;
-#pragma unroll
-    for (int j = 0; j < NX; j++) *reinterpret_cast<u32x4 *>(xs + xput + T / 8 * j * 128) = st.x[j];
+  auto put_w = [&](uint8_t *ws, const Stage &st) {
+    uint8_t *es = ws + WB;
 #pragma unroll
     for (int j = 0; j < NW; j++) {
       uint8_t *d = ws + wput + (T / CPR) * j * ROWB;
@@ -438,6 +521,12 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
       if constexpr (WT == XE_BFP16)
         *reinterpret_cast<uint16_t *>(es + (wr + (T / CPR) * j) * 8 + 2 * wc) = static_cast<uint16_t>(st.e[j]);
     }
+  };
+  auto put = [&](int buf, const Stage &st) {
+    uint8_t *xs = lds + buf;
+#pragma unroll
+    for (int j = 0; j < NX; j++) *reinterpret_cast<u32x4 *>(xs + xput + T / 8 * j * 128) = st.x[j];
+    put_w(xs + XB, st);
   };
 
   f32x16 acc[RX][RW][PA];
@@ -458,8 +547,8 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
   constexpr int QN = NB == 3 ? 2 : 1;
   uint32_t q[QN][RW][QW], ex[QN][RW];
   u32x4 wf[2][RW], xf[2][RX][P];
-  auto rdq = [&](int buf, uint32_t(&qv)[RW][QW], uint32_t(&ev)[RW]) {
-    const uint8_t *ws = lds + buf + XB, *es = ws + WB;
+  auto rdq_at = [&](const uint8_t *ws, uint32_t(&qv)[RW][QW], uint32_t(&ev)[RW]) {
+    const uint8_t *es = ws + WB;
     if constexpr (WT != XE_BF16)
 #pragma unroll
       for (int b = 0; b < RW; b++) {
@@ -471,6 +560,7 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
         if constexpr (WT == XE_BFP16) ev[b] = *reinterpret_cast<const uint32_t *>(es + (ww * 32 * RW + 32 * b + lr) * 8 + 4 * lh);
       }
   };
+  auto rdq = [&](int buf, uint32_t(&qv)[RW][QW], uint32_t(&ev)[RW]) { rdq_at(lds + buf + XB, qv, ev); };
   auto rdx = [&](int buf, int s, int d) {
     const uint8_t *xs = lds + buf, *ws = xs + XB;
 #pragma unroll
@@ -481,6 +571,88 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
     if constexpr (WT == XE_BF16)
 #pragma unroll
       for (int b = 0; b < RW; b++) wf[d][b] = *reinterpret_cast<const u32x4 *>(ws + (wget ^ (s << 4)) + 32 * b * ROWB);
+  };
+
+  // The steps in which a row of the tile has an fp32 block: every row as x 2^s
+  // in fp32 (which holds two parts exactly) and into three bf16 parts on its
+  // way to LDS (one buffer, two barriers a step), three MFMAs a product.
+  // Rare, so short code before speed: 13824 x 1152 x 512 rows, one call in a
+  // row of calls, 75 us with every step here, 50 with none.
+  auto raw_steps = [&](Stage &sj) {
+    constexpr int XR = 3 * BX * 128;
+    static_assert(P != 2 || XR + WB <= NB * BUF, "three row planes fit the operand buffers");
+    uint8_t *const ws = lds + XR;
+    const int steps = (K + kBK - 1) / kBK;
+    auto at = [&](int i) { return i < nsteps ? __builtin_amdgcn_readfirstlane(order[i]) : nsteps; };
+    int s1 = at(nfast);
+    issue_at(s1, sj);
+    for (int i1 = nfast; i1 < nsteps; i1++) {
+#pragma unroll
+      for (int j = 0; j < NX / 2; j++) {
+        const int r = xr + T / 8 * j, rw = rs[r];
+        const bool raw = n0 + r < p.n && rexp_raw(rw) && p.raw[raw_at(n0 + r, step0 + s1, steps)];
+        const f16x8 hi = __builtin_bit_cast(f16x8, sj.x[j]), lo = __builtin_bit_cast(f16x8, sj.x[j + NX / 2]);
+        float v[8], m[8], l[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          const uint32_t h = sj.x[j][i / 2], g = sj.x[j + NX / 2][i / 2];
+          const uint32_t w = i & 1 ? (h & 0xffff0000u) | g >> 16 : h << 16 | (g & 0xffffu);
+          v[i] = raw ? __builtin_ldexpf(__uint_as_float(w), rexp_s(rw))
+                     : static_cast<float>(hi[i]) + static_cast<float>(lo[i]) * (1.0f / (1 << kLoExp));
+          m[i] = v[i] - trunc_bf16(v[i]);
+          l[i] = m[i] - trunc_bf16(m[i]);
+        }
+        uint8_t *d = lds + xput + T / 8 * j * 128;
+        *reinterpret_cast<u32x4 *>(d) = u32x4{pack_hi16(v[0], v[1]), pack_hi16(v[2], v[3]), pack_hi16(v[4], v[5]), pack_hi16(v[6], v[7])};
+        *reinterpret_cast<u32x4 *>(d + BX * 128) = u32x4{pack_hi16(m[0], m[1]), pack_hi16(m[2], m[3]), pack_hi16(m[4], m[5]), pack_hi16(m[6], m[7])};
+        *reinterpret_cast<u32x4 *>(d + 2 * BX * 128) = u32x4{pack_hi16(l[0], l[1]), pack_hi16(l[2], l[3]), pack_hi16(l[4], l[5]), pack_hi16(l[6], l[7])};
+      }
+      put_w(ws, sj);
+      __syncthreads();
+      s1 = at(i1 + 1);
+      issue_at(s1, sj);
+      rdq_at(ws, q[0], ex[0]);
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        u32x4 w[RW];
+#pragma unroll
+        for (int b = 0; b < RW; b++)
+          w[b] = __builtin_bit_cast(u32x4, WT == XE_I8 ? i8_to_bf16(q[0][b][(2 * s) % QW], q[0][b][(2 * s + 1) % QW]) : i4_to_bf16(q[0][b][s % QW]));
+#pragma unroll
+        for (int pl = 0; pl < 3; pl++)
+#pragma unroll
+          for (int a = 0; a < RX; a++) {
+            const u32x4 xv = *reinterpret_cast<const u32x4 *>(lds + (xget ^ (s << 4)) + (pl * BX + 32 * a) * 128);
+#pragma unroll
+            for (int b = 0; b < RW; b++) acc[a][b][0] = mfma<XE_BF16>(w[b], xv, acc[a][b][0]);
+          }
+      }
+      __syncthreads();
+    }
+  };
+  // Which steps those are: order, nfast.
+  auto sort_steps = [&]() {
+    const int steps = (K + kBK - 1) / kBK;
+    for (int i = threadIdx.x; i < nsteps; i += T) hit[i] = 0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < nsteps * BX; i += T) {
+      const int r = i % BX, st = i / BX;
+      if (n0 + r < p.n && rexp_raw(rs[r]) && p.raw[raw_at(n0 + r, step0 + st, steps)]) hit[st] = 1;
+    }
+    __syncthreads();
+    if (wave == 0) {
+      int fast = 0;
+      for (int i0 = 0; i0 < nsteps; i0 += 64) {
+        const bool on = i0 + lane < nsteps, raw = on && hit[i0 + lane];
+        const uint64_t fm = __ballot(on && !raw), below = (uint64_t(1) << lane) - 1;
+        const int before = fast + __popcll(fm & below);  // steps without fp32 blocks before this one
+        if (on) order[raw ? nsteps - 1 - (i0 + lane - before) : before] = static_cast<uint8_t>(i0 + lane);
+        fast += __popcll(fm);
+      }
+      if (lane == 0) seen[8] = fast;
+    }
+    __syncthreads();
+    nfast = __builtin_amdgcn_readfirstlane(seen[8]);
   };
 
   // Step s.  The loads of step s + D (D = NB - 1) go from their registers to
@@ -494,7 +666,7 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
   Stage st[NS];
   int bc = 0, bp = D * BUF;  // LDS offset of the buffer of this step and of the one being filled
   auto nxt = [&](int b) { return b + BUF == NB * BUF ? 0 : b + BUF; };
-  auto step = [&](int j, int next_issue, auto more) {
+  auto step = [&](int j, int next_issue, auto more, auto sorted) {
     Stage &sj = st[(j + D) % NS];
     const int bn = nxt(bc);
     if constexpr (NB == 2) {
@@ -518,15 +690,20 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
           wf[s & 1][b] = __builtin_bit_cast(u32x4, bfp_to_bf16(qv[b][2 * s], qv[b][2 * s + 1], (ex[j % QN][b] >> (8 * s)) & 0xffu));
       }
 #pragma unroll
-      for (int pl = 0; pl < P; pl++)
+      for (int pl = 0; pl < P; pl++) {
+        if constexpr (P == 2 && PA == 1)  // else the second part's sums are scaled at the end
+          if (pl == 1)
+#pragma unroll
+            for (int b = 0; b < RW; b++) wf[s & 1][b] = lo_weights(wf[s & 1][b]);
 #pragma unroll
         for (int a = 0; a < RX; a++)
 #pragma unroll
           for (int b = 0; b < RW; b++)
             acc[a][b][pl % PA] = mfma<WT>(wf[s & 1][b], xf[s & 1][a][pl], acc[a][b][pl % PA]);
+      }
       if (s == 0) {
         put(bp, sj);
-        if constexpr (decltype(more)::value) issue(next_issue, sj);
+        if constexpr (decltype(more)::value) issue(next_issue, sj, sorted);
       }
     }
     __syncthreads();
@@ -534,11 +711,8 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
     bp = nxt(bp);
   };
 #pragma unroll
-  for (int j = 0; j < NS; j++) issue(j, st[j]);
-  // what the epilogue needs, loaded behind the first operands, in LDS: the
-  // rows' exponents, the weight rows' scales and biases
-  int *const rs = reinterpret_cast<int *>(lds + kEpi);
-  float *const wsc = reinterpret_cast<float *>(rs + BX), *const wbi = wsc + BW;
+  for (int j = 0; j < NS; j++) issue_at(j, st[j]);
+  // what the epilogue needs, loaded behind the first operands
   int t_rs = 0;
   float t_sc = 1.0f, t_bi = 0.0f;
   if constexpr (P == 2) t_rs = p.rexp[n0 + threadIdx.x % BX];
@@ -548,6 +722,12 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
     if (p.bias) t_bi = p.bias[m];
   }
   auto put_tables = [&]() {
+    if constexpr (P == 2) {
+      static_assert(kEarly && T / 64 <= 8, "the row exponents are in LDS before the K loop");
+      const bool mine = rexp_raw(t_rs) && n0 + static_cast<int>(threadIdx.x) % BX < p.n;
+      const bool any = __any(mine);
+      if (lane == 0) seen[wave] = any;
+    }
     if (threadIdx.x < BX) rs[threadIdx.x] = t_rs;
     if (threadIdx.x < BW) {
       wsc[threadIdx.x] = t_sc;
@@ -555,26 +735,48 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
     }
   };
   if constexpr (kEarly) put_tables();
+  auto fill = [&](auto sorted) {
 #pragma unroll
-  for (int d = 0; d < D; d++) {
-    put(d * BUF, st[d % NS]);
-    issue(d + NS, st[d % NS]);
-  }
-  __syncthreads();
-  if constexpr (NB == 3) {
-    rdx(0, 0, 0);
-    rdq(0, q[0], ex[0]);
-  }
+    for (int d = 0; d < D; d++) {
+      put(d * BUF, st[d % NS]);
+      issue(d + NS, st[d % NS], sorted);
+    }
+    __syncthreads();
+    if constexpr (NB == 3) {
+      rdx(0, 0, 0);
+      rdq(0, q[0], ex[0]);
+    }
+  };
   // whole groups of NS steps, so that every stage is a fixed set of
   // registers; the remainder's loads are in flight by then
-  int s0 = 0;
-  for (; s0 + NS <= nsteps; s0 += NS) {
+  auto fast_steps = [&](auto sorted) {
+    int s0 = 0;
+    for (; s0 + NS <= nfast; s0 += NS) {
 #pragma unroll
-    for (int j = 0; j < NS; j++) step(j, s0 + j + D + NS, std::true_type{});
+      for (int j = 0; j < NS; j++) step(j, s0 + j + D + NS, std::true_type{}, sorted);
+    }
+#pragma unroll
+    for (int j = 0; j < NS - 1; j++)
+      if (s0 + j < nfast) step(j, 0, std::false_type{}, sorted);
+  };
+  fill(std::false_type{});
+  bool fp32 = false;
+  if constexpr (P == 2) {
+    int any = 0;
+#pragma unroll
+    for (int i = 0; i < T / 64; i++) any |= seen[i];
+    fp32 = __builtin_amdgcn_readfirstlane(any) != 0;
   }
+  if (!fp32) {
+    fast_steps(std::false_type{});
+  } else if constexpr (P == 2) {
+    sort_steps();
 #pragma unroll
-  for (int j = 0; j < NS - 1; j++)
-    if (s0 + j < nsteps) step(j, 0, std::false_type{});
+    for (int j = 0; j < NS; j++) issue(j, st[j], std::true_type{});
+    fill(std::true_type{});
+    fast_steps(std::true_type{});
+    raw_steps(st[0]);
+  }
 
   // A lane's results: weight rows 8 (i / 4) + 4 (lane / 32) + i % 4 of row
   // lane % 32 of each block.  The epilogue in registers, then through the
@@ -589,7 +791,7 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
   for (int a = 0; a < RX; a++) {
     int sx = 0;
-    if constexpr (P == 2) sx = -rs[wx * 32 * RX + 32 * a + lr];
+    if constexpr (P == 2) sx = -rexp_s(rs[wx * 32 * RX + 32 * a + lr]);
     float *const orow = out + (32 * a + lr) * OS;
 #pragma unroll
     for (int b = 0; b < RW; b++)
@@ -601,7 +803,7 @@ __global__ __launch_bounds__(64 * WXN * WWN) __attribute__((amdgpu_waves_per_eu(
         for (int i = 0; i < 4; i++) {
           float t = acc[a][b][0][4 * i4 + i];
 #pragma unroll
-          for (int q = 1; q < PA; q++) t += acc[a][b][q][4 * i4 + i];
+          for (int q = 1; q < PA; q++) t += P == 2 ? acc[a][b][q][4 * i4 + i] * (1.0f / (1 << kLoExp)) : acc[a][b][q][4 * i4 + i];
           if constexpr (P == 2) t = __builtin_ldexpf(t, sx);
           v[i] = t;
         }
@@ -759,7 +961,7 @@ void rows_launch(const gdev::GemvParams &p, const WideRows &rows, hipStream_t s)
   const int nv = (p.k / 4 + kT - 1) / kT;
   auto fn = nv <= 1 ? wide_rows_kernel<1, P> : nv <= 2 ? wide_rows_kernel<2, P> : nv <= 4 ? wide_rows_kernel<4, P>
             : nv <= 8 ? wide_rows_kernel<8, P> : wide_rows_kernel<16, P>;
-  hipLaunchKernelGGL(fn, dim3(p.batch), dim3(kT), 0, s, p, rows.planes, rows.rexp);
+  hipLaunchKernelGGL(fn, dim3(p.batch), dim3(kT), 0, s, p, rows.planes, rows.rexp, rows.raw);
   XE_HIP(hipGetLastError());
 }
 
@@ -770,6 +972,7 @@ bool al16(const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
 int wide_planes(int wdtype) { return wdtype == XE_I8 || wdtype == XE_I4 ? 2 : 3; }
 size_t wide_plane_elems(int wdtype, int n, int k) { return static_cast<size_t>(wide_planes(wdtype)) * n * k; }
 size_t wide_rexp_ints(int n) { return (static_cast<size_t>(n) + kRowPad - 1) / kRowPad * kRowPad; }
+size_t wide_raw_ints(int n, int k) { return wide_rexp_ints(n) / 4 * ((k + kBK - 1) / kBK); }
 
 bool wide_takes(int m, int k, int n, int wdtype, const void *x, int ldx) {
   if (wdtype != XE_I8 && wdtype != XE_I4 && wdtype != XE_BF16 && wdtype != XE_BFP16) return false;
@@ -806,7 +1009,7 @@ void launch_wide_rows(const gdev::GemvParams &p, int wdtype, const WideRows &row
   XE_REQUIRE(!p.sub_part || (p.sub_ks >= 1 && p.sub_ks <= kMaxKs && p.sub_out_scale == 1.0f),
              "wide rows: too many split partials");
   if (wide_planes(wdtype) == 2) {
-    XE_REQUIRE(rows.rexp, "wide rows: row exponents missing");
+    XE_REQUIRE(rows.rexp && rows.raw, "wide rows: row exponents missing");
     rows_launch<2>(p, rows, s);
   } else {
     rows_launch<3>(p, rows, s);
@@ -815,7 +1018,7 @@ void launch_wide_rows(const gdev::GemvParams &p, int wdtype, const WideRows &row
 
 void launch_wide_gemm(const WideGemm &g, hipStream_t s) {
   XE_REQUIRE(wide_takes(g.m, g.k, g.n, g.wdtype, g.rows.planes, 0), "wide gemm: unsupported shape");
-  XE_REQUIRE((g.wdtype != XE_I8 && g.wdtype != XE_I4) || (g.scale && g.rows.rexp), "wide gemm: int8/int4 weight without scales");
+  XE_REQUIRE((g.wdtype != XE_I8 && g.wdtype != XE_I4) || (g.scale && g.rows.rexp && g.rows.raw), "wide gemm: int8/int4 weight without scales");
   XE_REQUIRE(g.wdtype != XE_BFP16 || g.exps, "wide gemm: bfp16 weight without exponents");
   XE_REQUIRE(g.act != ACT_GEGLU_TANH || (g.m % 4 == 0 && !g.pack), "wide gemm: GeGLU rows must pair within 4-row groups");
   XE_REQUIRE(!g.pack || (g.m % g.pack_hd == 0 && g.pack_hd % 4 == 0), "wide gemm: packed heads must hold whole quads");
@@ -832,6 +1035,7 @@ void launch_wide_gemm(const WideGemm &g, hipStream_t s) {
   p.n = g.n;
   p.planes = g.rows.planes;
   p.rexp = g.rows.rexp;
+  p.raw = g.rows.raw;
   p.act = g.act;
   p.y = g.y;
   p.ldy = g.ldy;

@@ -38,3 +38,26 @@ def test_grouped_merge(gpu, monkeypatch, hq, hkv, hd, ctxlen, b):
     assert np.array_equal(bits, np.asarray(again, np.float32).view(np.uint32))
     assert np.array_equal(bits, np.asarray(launched, np.float32).view(np.uint32))
     close(first, O.attn_decode(q, kc, vc, lens, scale))
+
+
+@pytest.mark.parametrize("hq,hkv,hd,ctxlen", [(4, 1, 256, 1088), (4, 1, 256, 4160), (8, 2, 128, 1100), (2, 2, 64, 3000)])
+def test_merge_of_infinite_values(gpu, monkeypatch, hq, hkv, hd, ctxlen):
+    """An infinity in the last split's values, with a split count that leaves
+    the last group short: infinite in that dimension, untouched in the others,
+    the same from both merges."""
+    _, ctx = gpu
+    print("[case] infinite value hq=%d hkv=%d hd=%d ctx=%d" % (hq, hkv, hd, ctxlen), flush=True)
+    rng = np.random.default_rng(hq + ctxlen)
+    q = rng.standard_normal((1, hq, hd)).astype(np.float32)
+    kc = O.bf16_bits(rng.standard_normal((1, hkv, ctxlen, hd)).astype(np.float32))
+    vc = O.bf16_bits(rng.standard_normal((1, hkv, ctxlen, hd)).astype(np.float32))
+    lens, scale = np.array([ctxlen], np.int32), 1.0 / math.sqrt(hd)
+    finite = O.attn_decode(q, kc, vc, lens, scale).reshape(hq, hd)
+    vc[0, :, ctxlen - 1, 5] = 0x7F80
+    vc[0, :, ctxlen - 1, 9] = 0xFF80
+    for merge in ("block", "launch"):
+        monkeypatch.setenv("XE_ATTN_MERGE", merge)
+        got = np.asarray(ctx.attn(q, kc, vc, lens, scale)).reshape(hq, hd)
+        assert np.all(got[:, 5] == np.inf) and np.all(got[:, 9] == -np.inf), merge
+        rest = np.delete(np.arange(hd), [5, 9])
+        close(got[:, rest], finite[:, rest])

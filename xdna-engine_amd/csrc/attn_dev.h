@@ -617,7 +617,7 @@ __device__ __forceinline__ void attn_merge_block(const AttnParams &p, int blk, i
 // 4 heads x 256 of one key head, one stream, split and merge, us: 32768 keys
 // 34.9 (256 threads, one level, at most 64 splits) -> 17.7, 4096 keys 16.6 ->
 // 11.7, 8 streams at 4096 keys 20.4 -> 15.3 (20.3 / 13.1 / 16.8 with a branch
-// a load instead of clamped loads at weight zero).
+// a load instead of clamped loads).
 constexpr int kTeams = 4;
 __host__ __device__ constexpr int team_threads(int hd, int g) { return g * hd < kThreads ? g * hd : kThreads; }
 template <int HD, int G>
@@ -646,7 +646,7 @@ __device__ __forceinline__ void attn_merge_wide(const AttnParams &p, int blk, in
   for (int j = 0; j < NG; j++) {
     const int s0 = (team + j * kTeams) * gs;
     if (s0 >= nsplits) continue;
-    // past the last split: that one again, with weight zero
+    // past the last split: that one again, not used
     auto ld = [&](int i) { v[j][i] = wbase[(hh * p.max_splits + min(s0 + i, nsplits - 1)) * RS + 2 + e]; };
 #pragma unroll
     for (int i = 0; i < kGroup / 2; i++) ld(i);
@@ -677,6 +677,11 @@ __device__ __forceinline__ void attn_merge_wide(const AttnParams &p, int blk, in
     const int grp = team + j * kTeams;
     if (grp >= groups) continue;
     float at0 = 0.f, at1 = 0.f;
+    const int n = nsplits - grp * gs;
+    if (n < gs)  // a short group: an infinite sum times a weight of zero would be NaN
+#pragma unroll
+      for (int i = 0; i < kGroup; i++)
+        if (i >= n) v[j][i] = 0.f;
     auto add = [&](int i) {
       if (i & 1) at1 += v[j][i] * wts[hh][grp][i];
       else at0 += v[j][i] * wts[hh][grp][i];

@@ -484,6 +484,13 @@ int xe_decoder_profile_step(xe_decoder *dec, int batch, int max_entries, char *l
  * reference (its executors are fixed per backend); returns -1 on error. */
 enum { XE_EXEC_GRAPH = 0, XE_EXEC_EAGER = 2, XE_EXEC_LL = 3 };
 int xe_decoder_executor(xe_decoder *dec, int batch);
+/* Tokens of a stream that one pass of feed / generate over a prompt of
+ * n_prompt tokens takes (whole layers over up to 2048 rows at once, whichever
+ * executor runs the steps); 0: the prompt is fed one step at a time on that
+ * executor -- one token, two of one stream, int8 cross K / V, or a workspace
+ * beyond XE_PROMPT_MB megabytes (unset: no limit; 0: always; a pass is made
+ * smaller first).  No counterpart in the reference; -1 on error. */
+int xe_decoder_prompt_pass(xe_decoder *dec, int batch, int n_prompt);
 /* Resident decode step (ElfResident, npu-xrt/src/lib.rs:591-629 and
  * xrt_shim.h:95-111: a constant program bound once, per-token parameters
  * written to a host-mapped scratchpad, then dispatched).  open() builds the

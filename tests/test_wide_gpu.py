@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 import oracle_lib as O
-from parity_util import compare_logits
+from parity_util import compare_logits, greedy_identity
 from test_decoder_gpu import build, prompts, tiny
 
 pytestmark = pytest.mark.gpu
@@ -86,6 +86,54 @@ def test_prompt_passes_logits(gpu, xe, family, wd, batch, n):
     for p in range(n):
         want = om.step(pr[:, p], np.full(batch, p, np.int32))
     compare_logits(got, want, "prompt-%s-%s-b%d-n%d" % (family, wd, batch, n))
+    dec.close()
+    om.close()
+
+
+@pytest.mark.parametrize("step", ["ll", "graph"])
+@pytest.mark.parametrize("family,batch", [("opt", 1), ("opt", 3), ("gemma", 1), ("gemma", 4), ("whisper", 2)])
+def test_prompt_without_a_workspace(gpu, xe, monkeypatch, step, family, batch):
+    """No room for a pass (a limit of nothing, as an allocation that fails):
+    the prompt is fed token by token on the step executor -- the low-latency
+    launch with its forced tokens, or the graph replayed -- and the streams go
+    on from there."""
+    monkeypatch.setenv("XE_STEP", step)
+    monkeypatch.setenv("XE_PROMPT_MB", "0")
+    cfg = prompt_cfg(xe, family, "i8")
+    print("[case] prompt without a workspace %s batch %d %s" % (family, batch, step), flush=True)
+    dec, om = build(xe, gpu, cfg, seed=37, batch=batch)
+    n = 7
+    assert dec.executor(batch) == step and dec.prompt_pass(batch, n) == 0
+    pr = prompts(cfg, batch, n, seed=4)
+    dec.feed(pr[:, :-1])
+    got, _ = dec.step(pr[:, -1], np.full(batch, n - 1, np.int32))
+    for p in range(n):
+        want = om.step(pr[:, p], np.full(batch, p, np.int32))
+    compare_logits(got, want, "prompt-steps-%s-b%d-%s" % (family, batch, step))
+    om.reset()
+    greedy_identity(dec.generate(pr, 12), om, pr, "prompt-steps-%s-b%d-%s" % (family, batch, step))
+    dec.close()
+    om.close()
+
+
+@pytest.mark.parametrize("family,batch,n,mb", [("gemma", 1, 75, "34"), ("gemma", 2, 330, "36"), ("gemma_hd128", 3, 41, "34.5"),
+                                               ("opt", 2, 90, "35"), ("whisper", 5, 31, "35")])
+def test_prompt_in_smaller_passes(gpu, xe, monkeypatch, family, batch, n, mb):
+    """A workspace limit that a pass over the whole prompt exceeds (as an
+    allocation that fails): smaller passes, the later ones over cached keys."""
+    monkeypatch.delenv("XE_STEP", raising=False)
+    cfg = prompt_cfg(xe, family, "i8")
+    print("[case] smaller passes %s batch %d, %d tokens, %s MB" % (family, batch, n, mb), flush=True)
+    dec, om = build(xe, gpu, cfg, seed=41, batch=batch)
+    assert dec.prompt_pass(batch, n - 1) == n - 1
+    monkeypatch.setenv("XE_PROMPT_MB", mb)
+    assert 2 <= dec.prompt_pass(batch, n - 1) < n - 1
+    pr = prompts(cfg, batch, n, seed=n)
+    dec.feed(pr[:, :-1])
+    got, _ = dec.step(pr[:, -1], np.full(batch, n - 1, np.int32))
+    for p in range(n):
+        want = om.step(pr[:, p], np.full(batch, p, np.int32))
+    compare_logits(got, want, "prompt-passes-%s-b%d-n%d" % (family, batch, n))
     dec.close()
     om.close()
 

@@ -1811,8 +1811,8 @@ struct PromptWs {
   bool wide;  // every linear suits the plane kernels (wide.hip)
 };
 
-// False where the device has no room for it.
-bool prompt_ws(xe_decoder *d, int rows, PromptWs &w) {
+// Its layout at `b`; returns the bytes it takes.
+size_t prompt_ws_layout(const xe_decoder *d, int rows, char *b, PromptWs &w) {
   const auto &c = d->c;
   const size_t D = c.d_model, hq = static_cast<size_t>(c.n_heads) * c.head_dim, R = rows;
   const int kmax = static_cast<int>(std::max(std::max(D, hq), static_cast<size_t>(c.ffn)));
@@ -1827,6 +1827,17 @@ bool prompt_ws(xe_decoder *d, int rows, PromptWs &w) {
   const size_t o_x0 = take(R * D), o_x1 = take(R * D), o_sub = take(R * D), o_qkv = take(R * d->nqkv());
   const size_t o_att = take(R * std::max(hq, D)), o_ffn = take(R * std::max(static_cast<size_t>(c.ffn), d->nqkv())), o_qx = take(R * D), o_rows = take(plane);
   const size_t o_part = take(gemm_ws_floats()), o_cnt = take(gemm_cnt_words()), o_tok = take(R), o_pos = take(R);
+  auto at = [&](size_t o) { return reinterpret_cast<float *>(reinterpret_cast<uintptr_t>(b) + o); };
+  w.x[0] = at(o_x0), w.x[1] = at(o_x1), w.sub = at(o_sub), w.qkv = at(o_qkv), w.att = at(o_att), w.ffn = at(o_ffn);
+  w.qx = at(o_qx), w.rows = at(o_rows), w.part = at(o_part), w.cnt = reinterpret_cast<unsigned *>(at(o_cnt));
+  w.wide = wide_takes(std::max(std::max(static_cast<int>(d->nqkv()), c.d_model), 2 * c.ffn), kmax, rows, c.wdtype, b, 0);
+  w.tok = reinterpret_cast<int32_t *>(at(o_tok)), w.pos = reinterpret_cast<int32_t *>(at(o_pos));
+  return off;
+}
+
+// False where the device has no room for it.
+bool prompt_ws(xe_decoder *d, int rows, PromptWs &w) {
+  const size_t off = prompt_ws_layout(d, rows, d->prompt_ws, w);
   if (off > d->prompt_ws_bytes) {
     XE_HIP(hipStreamSynchronize(d->s));
     if (d->prompt_ws) XE_HIP(hipFree(d->prompt_ws));
@@ -1840,13 +1851,8 @@ bool prompt_ws(xe_decoder *d, int rows, PromptWs &w) {
     }
     XE_HIP(e);
     d->prompt_ws_bytes = off;
+    (void)prompt_ws_layout(d, rows, d->prompt_ws, w);
   }
-  char *b = d->prompt_ws;
-  auto at = [&](size_t o) { return reinterpret_cast<float *>(b + o); };
-  w.x[0] = at(o_x0), w.x[1] = at(o_x1), w.sub = at(o_sub), w.qkv = at(o_qkv), w.att = at(o_att), w.ffn = at(o_ffn);
-  w.qx = at(o_qx), w.rows = at(o_rows), w.part = at(o_part), w.cnt = reinterpret_cast<unsigned *>(at(o_cnt));
-  w.wide = wide_takes(std::max(std::max(static_cast<int>(d->nqkv()), c.d_model), 2 * c.ffn), kmax, rows, c.wdtype, b, 0);
-  w.tok = reinterpret_cast<int32_t *>(at(o_tok)), w.pos = reinterpret_cast<int32_t *>(at(o_pos));
   return true;
 }
 
@@ -2039,7 +2045,8 @@ void prompt_chunk(xe_decoder *d, const PromptWs &w, int B, int t0, int t_n, bool
   XE_HIP(hipMemcpyAsync(d->xa, x, static_cast<size_t>(B) * D * 4, hipMemcpyDeviceToDevice, d->s));
 }
 
-// Whether feed() runs a prompt in passes instead of token by token.
+// Whether feed() runs a prompt in passes instead of token by token, where
+// there is memory for a pass.
 bool prompt_in_passes(xe_decoder *d, int batch, int n_prompt) {
   const auto &c = d->c;
   if (d->cross_i8k || d->cross_i8v) return false;  // int8 cross rows: the single-query kernels read them
@@ -2049,12 +2056,30 @@ bool prompt_in_passes(xe_decoder *d, int batch, int n_prompt) {
   return (n_prompt >= 3 || (n_prompt == 2 && batch >= 2)) && batch <= kPromptRows && prompt_attn_takes(c.head_dim, c.n_heads / c.n_kv_heads);
 }
 
-// The prompt in passes over up to kPromptRows rows; h: pinned staging.  False,
-// and nothing done, without memory for a pass.
+// Half the tokens a pass, for less memory; 0: one step at a time is as fast.
+int fewer_tokens(int tc) { return tc < 4 ? 0 : (tc + 1) / 2; }
+
+// Tokens of a stream that a pass over such a prompt takes (its workspace
+// within XE_PROMPT_MB megabytes, where that is set); 0: token by token.
+int prompt_pass_tokens(xe_decoder *d, int batch, int n_prompt) {
+  if (!prompt_in_passes(d, batch, n_prompt)) return 0;
+  int tc = std::max(1, std::min(n_prompt, kPromptRows / batch));
+  if (const char *e = std::getenv("XE_PROMPT_MB")) {
+    const double cap = std::atof(e) * 1e6;
+    PromptWs w{};
+    while (tc && static_cast<double>(prompt_ws_layout(d, batch * tc, nullptr, w)) > cap) tc = fewer_tokens(tc);
+  }
+  return tc;
+}
+
+// The prompt in passes over up to kPromptRows rows, fewer where there is no
+// memory for those; h: pinned staging.  False, and nothing done, where a
+// prompt of this size runs token by token.
 bool feed_passes(xe_decoder *d, const int32_t *prompt, int n_prompt, int batch, int32_t *h) {
-  const int tc = std::max(1, std::min(n_prompt, kPromptRows / batch));
+  int tc = prompt_pass_tokens(d, batch, n_prompt);
   PromptWs w{};
-  if (!prompt_ws(d, batch * tc, w)) return false;
+  while (tc && !prompt_ws(d, batch * tc, w)) tc = fewer_tokens(tc);
+  if (!tc) return false;
   XE_HIP(hipMemsetAsync(d->stop_dev + 1, 0, batch * 4, d->s));  // no stream has stopped
   XE_HIP(hipMemsetAsync(w.cnt, 0, gemm_cnt_words() * sizeof(unsigned), d->s));
   size_t at = 0;
@@ -2703,7 +2728,7 @@ void feed(xe_decoder *d, const int32_t *prompt, int n_prompt, int batch) {
   int32_t *h = d->host_tok;
   XE_REQUIRE(static_cast<size_t>(n_prompt + 1) * batch <= static_cast<size_t>(2) * (d->c.max_ctx + 2) * d->max_batch,
              "prompt too long for staging");
-  if (prompt_in_passes(d, batch, n_prompt) && feed_passes(d, prompt, n_prompt, batch, h)) {
+  if (feed_passes(d, prompt, n_prompt, batch, h)) {
     for (int b = 0; b < batch; b++) d->hpos[b] = n_prompt;
     d->live = batch;
     return;
@@ -3051,6 +3076,14 @@ int xe_decoder_executor(xe_decoder *d, int batch) {
       case Exec::Graph: break;
     }
     return XE_EXEC_GRAPH;
+  }, -1);
+}
+
+int xe_decoder_prompt_pass(xe_decoder *d, int batch, int n_prompt) {
+  return guard_d([&]() -> int {
+    XE_REQUIRE(d, "null decoder");
+    XE_REQUIRE(batch >= 1 && batch <= d->max_batch && n_prompt >= 1, "batch or prompt out of range");
+    return prompt_pass_tokens(d, batch, n_prompt);
   }, -1);
 }
 

@@ -52,6 +52,7 @@ EXPORTS = [
     "xe_decoder_generate", "xe_decoder_last_step_us", "xe_decoder_weight_bytes", "xe_decoder_set_stop",
     "xe_decoder_generate_until",
     "xe_decoder_feed", "xe_decoder_decode", "xe_decoder_profile_step", "xe_decoder_executor",
+    "xe_decoder_prompt_pass",
     "xe_model_tensor_shape", "xe_decoder_config", "xe_decoder_load_safetensors", "xe_safetensors_plan",
     "xe_ctx_record", "xe_run_query", "xe_run_wait", "xe_run_free", "xe_resident_open", "xe_resident_close",
     "xe_resident_write", "xe_resident_dispatch", "xe_resident_dispatch_start", "xe_resident_read",
@@ -176,6 +177,7 @@ def lib():
         "xe_decoder_profile_step": (i, [vp, i, i, vp, vp, vp]),
         "xe_decoder_weight_bytes": (u64, [vp]),
         "xe_decoder_executor": (i, [vp, i]),
+        "xe_decoder_prompt_pass": (i, [vp, i, i]),
         "xe_ctx_record": (vp, [vp]),
         "xe_run_query": (i, [vp]),
         "xe_run_wait": (i, [vp]),
@@ -683,6 +685,10 @@ class Decoder:
         """Name of the executor a step of `batch` streams runs on."""
         b = batch or self.batch or 1
         return EXECUTORS[_check(lib().xe_decoder_executor(self.h, b))]
+
+    def prompt_pass(self, batch, n_prompt):
+        """Tokens of a stream a pass over such a prompt takes (0: fed step by step)."""
+        return _check(lib().xe_decoder_prompt_pass(self.h, batch, n_prompt))
 
     def last_step_us(self):
         return lib().xe_decoder_last_step_us(self.h)

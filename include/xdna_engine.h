@@ -200,6 +200,21 @@ int xe_fused_norm_gemv(xe_ctx *ctx, const xe_weight *w, const void *x,
 int xe_gemv_dev(xe_ctx *ctx, const xe_weight *w, const void *x_dev,
                 int x_dtype, int batch, float *y_dev);
 
+/* Kernel that xe_gemv / xe_fused_norm_gemv run a shape on (16-byte aligned
+ * activations), by the same rule: the bandwidth GEMV, the MFMA GEMM that
+ * splits the fp32 rows in its tiles, or the one over row planes made once a
+ * row, in tiles of 64 x 64 or 128 rows x 256 weight rows; k_splits (may be
+ * NULL) receives the K splits of the latter two, else 0.  No device work.
+ * No counterpart in the reference; -1 on error. */
+enum xe_linear_kernel {
+  XE_LINEAR_GEMV = 0,
+  XE_LINEAR_GEMM = 1,
+  XE_LINEAR_PLANES = 2,
+  XE_LINEAR_PLANES_BIG = 3
+};
+int xe_linear_path(int wdtype, int m, int k, int norm, int x_dtype, int batch,
+                   int *k_splits);
+
 /* int8 activations x int8 weights -> int32 (ctx2.rs:771-830 device part):
  * acc[b,m] = sum_k xq[b,k] * q[m,k], exact.  w must be XE_I8; batch 1..512
  * (<= 8 rows an sdot4 GEMV, more the int8 MFMA GEMM). */

@@ -3,8 +3,10 @@ in passes over all their tokens.
 
 The GEMM is compared with a float64 product of the same stored weights
 (bar: rel-L2 1e-6, an fp32 sum's rounding at these K: about 2^-24 sqrt(K) / 4),
-at sizes that leave remainders in every tile: rows modulo 64 and 128, weight
-rows modulo 64 and 256, K modulo 64.  Prompts are compared with the oracle's
+at sizes that leave remainders in the tile that takes them (rows modulo 128 or
+64, weight rows modulo 256 or 64, K modulo 64): test_wide_linear on the 128 x
+256 tile (1153 x 6928 in bf16 / bfp16 on the GEMM without planes),
+test_wide_linear_paths on each tile, split and not.  Prompts are compared with the oracle's
 token-by-token logits (the bars of parity_util), at row counts either side of
 the plane kernels' first one, over several key tiles and over more rows than
 one pass takes.
@@ -61,6 +63,26 @@ def test_wide_linear(gpu, xe, wd, m, k, b, norm):
     # row by row: a row's exponent, padding or order mixed up shows here
     rows = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
     assert rows.max() <= 2e-6, "row %d rel-L2 %g" % (rows.argmax(), rows.max())
+
+
+# (kernel, K splits) a shape has to run on: both tiles, split and not, weight
+# counts that are odd, K beyond what one float4 round of 8 holds, the smallest
+PATHS = [
+    (4590, 640, 475, "ln", "i8 i4 bf16 bfp16", ("planes", 1)),
+    (3129, 2032, 127, "ln", "i8 i4", ("planes", 2)),
+    (1459, 9152, 126, "rms1p", "i8 i4", ("planes", 5)),
+    (21, 176, 77, "ln", "i8 i4 bf16 bfp16", ("planes", 1)),
+    (9969, 2192, 281, "rms1p", "i8 i4 bf16 bfp16", ("planes_big", 2)),
+    (3519, 8640, 133, "ln", "i8 i4 bf16 bfp16", ("planes_big", 8)),
+]
+
+
+@pytest.mark.parametrize("wd,m,k,b,norm,path", [(wd,) + c[:4] + (c[5],) for c in PATHS for wd in c[4].split()])
+def test_wide_linear_paths(gpu, xe, wd, m, k, b, norm, path):
+    wdtype = {"i8": xe.XE_I8, "i4": xe.XE_I4, "bf16": xe.XE_BF16, "bfp16": xe.XE_BFP16}[wd]
+    code = {"ln": xe.XE_NORM_LN, "rms1p": xe.XE_NORM_RMS1P}[norm]
+    assert xe.linear_path(wdtype, m, k, b, norm=code) == path
+    test_wide_linear(gpu, xe, wd, m, k, b, norm)
 
 
 def prompt_cfg(xe, family, wd):
@@ -149,6 +171,7 @@ def test_wide_linear_range_within_a_row(gpu, xe, wd, m, k, b):
     the sum of their magnitudes (n roundings of an fp32 sum, operands to
     2^-23 each, the scale)."""
     _, ctx = gpu
+    assert xe.linear_path(xe.XE_I8 if wd == "i8" else xe.XE_I4, m, k, b) == (("planes_big", 3) if m == 4100 else ("planes", 1))
     print("[case] wide range %s m=%d k=%d b=%d" % (wd, m, k, b), flush=True)
     rng = np.random.default_rng(m + b)
     x = rng.standard_normal((b, k)).astype(np.float32)

@@ -787,6 +787,25 @@ int xe_gemv_i8act_dev(xe_ctx *ctx, const xe_weight *w, const int8_t *xq_dev, int
   }, -1);
 }
 
+int xe_linear_path(int wdtype, int m, int k, int norm, int x_dtype, int batch, int *k_splits) {
+  return guard([&]() -> int {
+    XE_REQUIRE(m > 0 && k > 0 && k % 16 == 0 && batch >= 1 && batch <= kMaxOpBatch, "bad shape");
+    XE_REQUIRE(x_dtype == XE_F32 || x_dtype == XE_BF16, "x must be XE_F32 or XE_BF16");
+    GemvLaunch L;
+    L.wdtype = wdtype;
+    L.m = m;
+    L.k = L.ldx = k;
+    L.x_dtype = x_dtype;
+    L.batch = batch;
+    L.norm = norm;
+    L.ldy = m;
+    int ks = 0;
+    const int kernel = gemm_preferred(m, k, batch) ? gemm_op_kernel(L, &ks) : XE_LINEAR_GEMV;
+    if (k_splits) *k_splits = ks;
+    return kernel;
+  }, -1);
+}
+
 int xe_gemv_i8act(xe_ctx *ctx, const xe_weight *w, const int8_t *xq, int batch, int32_t *acc) {
   return guard([&]() -> int {
     XE_REQUIRE(ctx && w && xq && acc, "null argument");

@@ -169,6 +169,8 @@ void launch_gemm_op(const GemvLaunch &L, float *xn, float *ws, unsigned *cnt, hi
 // GEMM (gemm.hip) instead of the GEMV.
 bool gemm_preferred(int m, int k, int batch);
 size_t gemm_op_xn_floats(const GemvLaunch &L);
+// The GEMM it runs on (enum xe_linear_kernel) and, over planes, its K splits.
+int gemm_op_kernel(const GemvLaunch &L, int *k_splits);
 size_t gemm_op_ws_floats();
 size_t gemm_op_cnt_words();
 // Output of an int8 x int8 -> i32 product: the raw accumulator (acc set), or

@@ -1473,6 +1473,13 @@ size_t gemm_op_xn_floats(const GemvLaunch &L) {
   return gemm_needs_prologue(gdev::to_params(L)) ? static_cast<size_t>(L.batch) * L.k : 0;
 }
 
+int gemm_op_kernel(const GemvLaunch &L, int *k_splits) {
+  const bool wide = op_wide(L);
+  *k_splits = wide ? wide_splits(L.m, L.k, L.batch, L.wdtype, kGemmWsFloats) : 0;
+  if (!wide) return XE_LINEAR_GEMM;
+  return wide_big_tile(L.m, L.k, L.batch, L.wdtype, kGemmWsFloats) ? XE_LINEAR_PLANES_BIG : XE_LINEAR_PLANES;
+}
+
 void launch_gemm_op(const GemvLaunch &L, float *xn, float *ws, unsigned *cnt, hipStream_t s) {
   XE_REQUIRE(L.x_dtype == XE_F32 || L.x_dtype == XE_BF16, "gemm: fp32 or bf16 activations");
   gdev::GemvParams p = gdev::to_params(L);

@@ -68,6 +68,8 @@ bool wide_takes(int m, int k, int n, int wdtype, const void *x, int ldx);
 bool wide_preferred(int m, int k, int n, int wdtype, bool prologue);
 // K splits wide_gemm takes for a shape, with at most ws_floats floats of partials.
 int wide_splits(int m, int k, int n, int wdtype, size_t ws_floats);
+// Whether its tiles are the 128 x 256 ones (else 64 x 64).
+bool wide_big_tile(int m, int k, int n, int wdtype, size_t ws_floats);
 // x (+ sub, post norm, norm) of n rows -> planes; the fields x, x_bf16, ldx,
 // batch, k, sub, sub_part .., post_w, res_out, norm, gamma, beta, eps of p.
 void launch_wide_rows(const gdev::GemvParams &p, int wdtype, const WideRows &rows, hipStream_t s);

@@ -1001,6 +1001,10 @@ int wide_splits(int m, int k, int n, int wdtype, size_t ws_floats) {
   return choose_shape(m, k, n, wdtype, ws_floats).ks;
 }
 
+bool wide_big_tile(int m, int k, int n, int wdtype, size_t ws_floats) {
+  return choose_shape(m, k, n, wdtype, ws_floats).big;
+}
+
 void launch_wide_rows(const gdev::GemvParams &p, int wdtype, const WideRows &rows, hipStream_t s) {
   XE_REQUIRE(p.k % 16 == 0 && p.k <= kMaxK && p.batch > 0, "wide rows: unsupported shape");
   XE_REQUIRE(al16(p.x) && p.ldx % 4 == 0 && al16(p.sub) && al16(p.sub_part) && al16(p.post_w) && al16(p.res_out) &&

@@ -31,6 +31,7 @@ XE_NORM_NONE, XE_NORM_LN, XE_NORM_RMS, XE_NORM_RMS1P = 0, 1, 2, 3
 XE_LAYOUT_MK, XE_LAYOUT_KN = 0, 1
 XE_OPT, XE_WHISPER, XE_GEMMA3 = 0, 1, 2
 EXECUTORS = {0: "graph", 2: "eager", 3: "ll"}
+LINEAR_KERNELS = ("gemv", "gemm", "planes", "planes_big")  # enum xe_linear_kernel
 
 EXPORTS = [
     "xe_last_error", "xe_abi_version", "xe_device_count", "xe_device_open", "xe_device_close",
@@ -52,7 +53,7 @@ EXPORTS = [
     "xe_decoder_generate", "xe_decoder_last_step_us", "xe_decoder_weight_bytes", "xe_decoder_set_stop",
     "xe_decoder_generate_until",
     "xe_decoder_feed", "xe_decoder_decode", "xe_decoder_profile_step", "xe_decoder_executor",
-    "xe_decoder_prompt_pass",
+    "xe_decoder_prompt_pass", "xe_linear_path",
     "xe_model_tensor_shape", "xe_decoder_config", "xe_decoder_load_safetensors", "xe_safetensors_plan",
     "xe_ctx_record", "xe_run_query", "xe_run_wait", "xe_run_free", "xe_resident_open", "xe_resident_close",
     "xe_resident_write", "xe_resident_dispatch", "xe_resident_dispatch_start", "xe_resident_read",
@@ -178,6 +179,7 @@ def lib():
         "xe_decoder_weight_bytes": (u64, [vp]),
         "xe_decoder_executor": (i, [vp, i]),
         "xe_decoder_prompt_pass": (i, [vp, i, i]),
+        "xe_linear_path": (i, [i, i, i, i, i, i, C.POINTER(i)]),
         "xe_ctx_record": (vp, [vp]),
         "xe_run_query": (i, [vp]),
         "xe_run_wait": (i, [vp]),
@@ -550,6 +552,13 @@ class Resident:
         if self.h:
             lib().xe_resident_close(self.h)
             self.h = None
+
+
+def linear_path(wdtype, m, k, batch, norm=XE_NORM_NONE, x_dtype=XE_F32):
+    """(kernel a linear of this shape runs on, its K splits over row planes)."""
+    ks = C.c_int(0)
+    kernel = _check(lib().xe_linear_path(wdtype, m, k, norm, x_dtype, batch, C.byref(ks)))
+    return LINEAR_KERNELS[kernel], ks.value
 
 
 def tensor_shape(cfg, kind, layer):

@@ -261,14 +261,22 @@ int xe_attn_decode_dev(xe_ctx *ctx, const float *q_dev, const uint16_t *kc_dev,
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
  * split partials go to a static per-GPU workspace of 4 Mi floats (16 MB)
  * instead of the ctx's own; a call needing more (batch * hq * splits *
- * (hd + 2) floats, splits <= 64, or up to 256 while batch * hkv * splits <=
- * 512) fails with -1.  Same results as xe_attn_decode_dev.  Calls that overlap on one GPU (any ctx, any
+ * (hd + 2) floats, splits as xe_attn_splits says) fails with -1.  Same
+ * results as xe_attn_decode_dev.  Calls that overlap on one GPU (any ctx, any
  * thread) share the workspace and race: serialise them. */
 int xe_attn_decode_dev_static(xe_ctx *ctx, const float *q_dev,
                               const uint16_t *kc_dev, const uint16_t *vc_dev,
                               const int32_t *lens_dev, int batch, int hq,
                               int hkv, int hd, int max_ctx, float scale,
                               float *out_dev);
+
+/* Most key ranges that the attention calls above split a stream into: up to
+ * 64, or up to 256 while batch * hkv * splits <= 512 (256 with 8 query heads
+ * a key head).  merge_launch (may be NULL): 1 if xe_attn_decode[_dev] merges
+ * them in a launch of its own.  No counterpart in the reference; -1 on
+ * error. */
+int xe_attn_splits(const xe_ctx *ctx, int batch, int hq, int hkv, int hd,
+                   int max_ctx, int *merge_launch);
 
 /* Wait for the ctx stream; returns 0 or -1. */
 int xe_ctx_synchronize(xe_ctx *ctx);

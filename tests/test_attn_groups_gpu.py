@@ -61,3 +61,28 @@ def test_merge_of_infinite_values(gpu, monkeypatch, hq, hkv, hd, ctxlen):
         assert np.all(got[:, 5] == np.inf) and np.all(got[:, 9] == -np.inf), merge
         rest = np.delete(np.arange(hd), [5, 9])
         close(got[:, rest], finite[:, rest])
+
+
+@pytest.mark.parametrize("hq,hkv,hd", [(4, 1, 256), (8, 1, 64), (16, 2, 64), (8, 1, 256), (8, 2, 128), (12, 12, 64)])
+def test_splits_fit_the_chip(gpu, hq, hkv, hd):
+    """More than 64 splits a stream only while all workgroups are resident: two
+    a CU, one where 8 query heads share a key head (a second round of
+    workgroups took 8 x 64 at 9000 keys of two streams from 28.5 to 34.5 us);
+    512 outputs a key head merge in a launch beyond one group of splits."""
+    _, ctx = gpu
+    resident = 256 if hq // hkv == 8 else 512
+    for b in (1, 2, 3, 5, 16, 64):
+        for n in (1, 64, 65, 1024, 1025, 9000, 32768, 1 << 17):
+            splits, launch = ctx.attn_splits(b, hq, hkv, hd, n)
+            assert 1 <= splits <= min(256, -(-n // 64))
+            assert splits <= 64 or splits * b * hkv <= resident
+            outs = hq // hkv * hd
+            assert launch == (splits > 1 and (outs > 512 or (outs == 512 and splits > 16)))
+    print("[case] resident splits %d/%d x %d" % (hq, hkv, hd), flush=True)
+    rng = np.random.default_rng(hq + hd)
+    n = 9000
+    q = rng.standard_normal((2, hq, hd)).astype(np.float32)
+    kc = O.bf16_bits(rng.standard_normal((2, hkv, n, hd)).astype(np.float32))
+    vc = O.bf16_bits(rng.standard_normal((2, hkv, n, hd)).astype(np.float32))
+    lens = np.array([n, 5000], np.int32)
+    close(ctx.attn(q, kc, vc, lens, 0.1), O.attn_decode(q, kc, vc, lens, 0.1))

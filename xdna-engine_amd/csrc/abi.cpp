@@ -866,13 +866,15 @@ int xe_w8a8_linear(xe_ctx *ctx, const xe_weight *w, const float *x, int batch, f
 
 // Splits per (stream, kv head): about XE_ATTN_WG_PER_CU (default 2)
 // workgroups per CU in total, at most one per 64 cache rows and at most 64, or
-// 256 while the total stays within 2 a CU (so a few streams fill the chip, and
-// the partials beyond 64 splits fit the static workspace: at most 512 x 8
-// heads x 258 floats).
+// 256 while the CUs hold them all at once (so a few streams fill the chip, and
+// the partials beyond 64 splits fit the static workspace: at most 512 x 4
+// heads x 258 floats).  A CU holds two, of 8 query heads a key head one (286
+// registers): 8 x 64 on one key head, two streams, 9000 keys, us with 64
+// splits 28.4, 128 20.4, 141 30.0 (the latter two merged in a launch).
 // With the merge inside the split kernel, 2 a CU against 4 (graph replays,
 // config 3): GQA 4q/1kv x 256 b = 64 ctx 4096 52.3 / 58.3 us, b = 16 ctx
 // 4096 33.0 / 47.1, b = 64 ctx 1024 26.2 / 37.2; ctx 32768 within 4 %.
-static int attn_splits(const xe_ctx *ctx, int batch, int hkv, int max_ctx) {
+static int attn_splits(const xe_ctx *ctx, int batch, int hq, int hkv, int max_ctx) {
   static const int per_cu = [] {
     const char *e = std::getenv("XE_ATTN_WG_PER_CU");
     return e && std::atoi(e) > 0 ? std::atoi(e) : 2;
@@ -882,7 +884,7 @@ static int attn_splits(const xe_ctx *ctx, int batch, int hkv, int max_ctx) {
   const int cap = (max_ctx + 63) / 64;
   ms = ms < 1 ? 1 : ms;
   ms = ms > cap ? cap : ms;
-  const int top = std::min(256, std::max(64, 512 / (batch * hkv)));
+  const int top = std::min(256, std::max(64, (hq / hkv == 8 ? 256 : 512) / (batch * hkv)));
   return ms > top ? top : ms;
 }
 
@@ -891,18 +893,20 @@ static int attn_splits(const xe_ctx *ctx, int batch, int hkv, int max_ctx) {
 // counters where the split kernel merges in place (the last split block of a
 // (stream, kv head) to arrive merges its partials, one launch).  A caller's
 // workspace (the allocation-free entry point) takes the separate merge launch.
-// In place up to 512 outputs a (stream, kv head): its one block has all of
-// them to merge, past the L2; a launch gives every 256 outputs a block of up
-// to 1024 threads and plain loads.  us in place / launched: 4 heads x 256 of
-// one key head, one stream, 32768 keys 25.3 / 17.7, 4096 keys 15.6 / 11.7, 8
-// streams at 4096 19.0 / 15.3, 64 at 4096 52 / 50.3; 8 x 128 of two key heads,
-// two streams at 9000 keys 16.8 / 15.1 (the line lies above it: one size only);
-// 12 x 64, two streams at 4096 keys 9.1 / 10.0, one at 448 6.6 / 7.7.
+// In place below 512 outputs a (stream, kv head), and at 512 up to 16 splits
+// (one group): its one block has all of them to merge, past the L2; a launch
+// gives every 256 outputs a block of up to 1024 threads and plain loads.  us
+// in place / launched: 4 heads x 256 of one key head, one stream, 32768 keys
+// 25.3 / 18.2, 4096 keys 15.6 / 11.7, 8 streams at 4096 19.0 / 15.3, 64 at
+// 4096 52 / 50.3; 512 outputs (8 x 64 of one key head, 8 x 128 of two, 4 x 256
+// of two), one stream: 1100 keys 22.7 / 19.6, 9000 keys 25.9 / 21.6, 19.9 /
+// 17.7 and 18.7 / 16.6; 4 x 64 of one, 32768 keys 19.1 / 19.7; 12 x 64, two
+// streams at 4096 keys 9.1 / 10.0, one at 448 6.6 / 7.7.
 // XE_ATTN_MERGE=launch or =block selects one for the ctx workspace.
-static bool attn_merge_in_place(int outs) {
+static bool attn_merge_in_place(int outs, int splits) {
   const char *e = std::getenv("XE_ATTN_MERGE");
   if (e && std::string(e) == "launch") return false;
-  return (e && std::string(e) == "block") || outs <= 512;
+  return (e && std::string(e) == "block") || outs < 512 || (outs == 512 && splits <= 16);
 }
 
 static int attn_impl(xe_ctx *ctx, const float *q, const uint16_t *kc, const uint16_t *vc,
@@ -921,11 +925,11 @@ static int attn_impl(xe_ctx *ctx, const float *q, const uint16_t *kc, const uint
   a.scale = scale;
   a.lens = lens;
   a.out = out;
-  a.max_splits = attn_splits(ctx, batch, hkv, max_ctx);
+  a.max_splits = attn_splits(ctx, batch, hq, hkv, max_ctx);
   if (work) {
     a.work = work;
   } else {
-    const bool in_place = attn_merge_in_place(hq / hkv * hd);
+    const bool in_place = attn_merge_in_place(hq / hkv * hd, a.max_splits);
     ctx->ensure_attn(attn_work_floats(batch, hq, hd, a.max_splits),
                      in_place ? attn_cnt_words(batch, hkv) : 0);
     a.work = ctx->attn_work;
@@ -955,7 +959,7 @@ int xe_attn_decode_dev_static(xe_ctx *ctx, const float *q_dev, const uint16_t *k
     XE_REQUIRE(ctx && q_dev && kc_dev && vc_dev && lens_dev && out_dev, "null argument");
     XE_REQUIRE(batch > 0 && hq > 0 && hkv > 0 && hd > 0, "bad shape");
     DeviceGuard dg(ctx->dev->ordinal);
-    const size_t need = attn_work_floats(batch, hq, hd, attn_splits(ctx, batch, hkv, max_ctx));
+    const size_t need = attn_work_floats(batch, hq, hd, attn_splits(ctx, batch, hq, hkv, max_ctx));
     XE_REQUIRE(need <= attn_static_floats(),
                "xe_attn_decode_dev_static: " + std::to_string(need) + " partial floats needed, the static "
                "workspace holds " + std::to_string(attn_static_floats()) +
@@ -1119,6 +1123,16 @@ int xe_probe_gemv(xe_ctx *ctx, const xe_weight *const *ws, int n_weights, const 
   }, -1);
 }
 
+int xe_attn_splits(const xe_ctx *ctx, int batch, int hq, int hkv, int hd, int max_ctx, int *merge_launch) {
+  return guard([&]() -> int {
+    XE_REQUIRE(ctx, "null ctx");
+    XE_REQUIRE(batch > 0 && hq > 0 && hkv > 0 && hd > 0 && max_ctx > 0, "bad shape");
+    const int splits = attn_splits(ctx, batch, hq, hkv, max_ctx);
+    if (merge_launch) *merge_launch = splits > 1 && !attn_merge_in_place(hq / hkv * hd, splits) ? 1 : 0;
+    return splits;
+  }, -1);
+}
+
 int xe_probe_attn(xe_ctx *ctx, const float *q_dev, const uint16_t *kc_dev, const uint16_t *vc_dev,
                   const int32_t *lens_dev, int batch, int hq, int hkv, int hd, int max_ctx,
                   float scale, float *out_dev, int reps, int flags, double *us_per_call) {
@@ -1126,8 +1140,9 @@ int xe_probe_attn(xe_ctx *ctx, const float *q_dev, const uint16_t *kc_dev, const
     XE_REQUIRE(ctx && q_dev && kc_dev && vc_dev && lens_dev && out_dev && us_per_call, "null argument");
     XE_REQUIRE(batch > 0 && hq > 0 && hkv > 0 && hd > 0 && reps > 0, "bad shape");
     DeviceGuard dg(ctx->dev->ordinal);
-    ctx->ensure_attn(attn_work_floats(batch, hq, hd, attn_splits(ctx, batch, hkv, max_ctx)),
-                     attn_merge_in_place(hq / hkv * hd) ? attn_cnt_words(batch, hkv) : 0);  // no allocation under capture
+    const int splits = attn_splits(ctx, batch, hq, hkv, max_ctx);
+    ctx->ensure_attn(attn_work_floats(batch, hq, hd, splits),
+                     attn_merge_in_place(hq / hkv * hd, splits) ? attn_cnt_words(batch, hkv) : 0);  // no allocation under capture
     *us_per_call = time_captured(ctx, reps, flags, [&]() {
       attn_impl(ctx, q_dev, kc_dev, vc_dev, lens_dev, batch, hq, hkv, hd, max_ctx, scale, out_dev);
     });

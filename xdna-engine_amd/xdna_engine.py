@@ -53,7 +53,7 @@ EXPORTS = [
     "xe_decoder_generate", "xe_decoder_last_step_us", "xe_decoder_weight_bytes", "xe_decoder_set_stop",
     "xe_decoder_generate_until",
     "xe_decoder_feed", "xe_decoder_decode", "xe_decoder_profile_step", "xe_decoder_executor",
-    "xe_decoder_prompt_pass", "xe_linear_path",
+    "xe_decoder_prompt_pass", "xe_linear_path", "xe_attn_splits",
     "xe_model_tensor_shape", "xe_decoder_config", "xe_decoder_load_safetensors", "xe_safetensors_plan",
     "xe_ctx_record", "xe_run_query", "xe_run_wait", "xe_run_free", "xe_resident_open", "xe_resident_close",
     "xe_resident_write", "xe_resident_dispatch", "xe_resident_dispatch_start", "xe_resident_read",
@@ -179,6 +179,7 @@ def lib():
         "xe_decoder_weight_bytes": (u64, [vp]),
         "xe_decoder_executor": (i, [vp, i]),
         "xe_decoder_prompt_pass": (i, [vp, i, i]),
+        "xe_attn_splits": (i, [vp, i, i, i, i, i, C.POINTER(i)]),
         "xe_linear_path": (i, [i, i, i, i, i, i, C.POINTER(i)]),
         "xe_ctx_record": (vp, [vp]),
         "xe_run_query": (i, [vp]),
@@ -430,6 +431,12 @@ class CtxDecode:
         _check(lib().xe_probe_gemv(self.h, arr, len(weights), x_ptr, x_dtype, batch, y_ptr, reps,
                                    1 if eager else 0, C.byref(us)))
         return us.value
+
+    def attn_splits(self, b, hq, hkv, hd, max_ctx):
+        """(key ranges a stream splits into at most, whether a launch of its own merges them)."""
+        launch = C.c_int(0)
+        n = _check(lib().xe_attn_splits(self.h, b, hq, hkv, hd, max_ctx, C.byref(launch)))
+        return n, bool(launch.value)
 
     def probe_attn(self, q_ptr, k_ptr, v_ptr, lens_ptr, b, hq, hkv, hd, max_ctx, scale, out_ptr,
                    reps, eager=False):

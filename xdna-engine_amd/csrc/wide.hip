@@ -43,7 +43,7 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kT = 256;
 constexpr int kBK = 64;             // k per step
 constexpr int kNoRec = 0x7ffffff0;  // past every buffer: loads return zeros
-constexpr int kMaxK = 16384;        // rows kernel: 16 float4 a thread
+constexpr int kMaxK = 16384;        // rows kernel: 8 float4 a thread of 512
 constexpr int kMaxKs = 8;           // K splits
 constexpr int kRowPad = 128;        // rexp is readable up to a multiple of it
 constexpr int kLds = 160 * 1024;    // LDS of a CU
@@ -79,16 +79,16 @@ __device__ __forceinline__ float trunc_bf16(float x) { return __uint_as_float(__
 __device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
 
 // One workgroup a row: t = x (+ post(sub)) -> res_out, h = norm(t) -> planes.
-// A thread holds float4 chunks threadIdx.x + 256 j, j < NV, from the first
-// load to the plane stores (K <= 1024 NV), so the row is read once.  Bound by
+// A thread holds float4 chunks threadIdx.x + T j, j < NV, from the first load
+// to the plane stores (K <= 4 T NV), so the row is read once.  Bound by
 // its chain of block reductions (one per norm statistic, one for the row's
 // largest and smallest |h|), which the other rows' workgroups of the CU
 // overlap.
-template <int NV, int P>
-__global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint16_t *planes, int *rexp, uint8_t *raw_flags) {
+template <int NV, int P, int T>
+__global__ __launch_bounds__(T) void wide_rows_kernel(gdev::GemvParams p, uint16_t *planes, int *rexp, uint8_t *raw_flags) {
   __shared__ float red[2 * 4 * gdev::kMaxWaves];
-  __shared__ float mx[kT / 64];
-  __shared__ float mn[kT / 64];
+  __shared__ float mx[T / 64];
+  __shared__ float mn[T / 64];
   const int b = blockIdx.x, K = p.k, K4 = K / 4;
   const float fk = static_cast<float>(K);
   float t[NV][4], g[NV][4], be[NV][4];
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint1
   float su[NV][4], pw[NV][4];
 #pragma unroll
   for (int j = 0; j < NV; j++) {
-    const int i = 4 * (static_cast<int>(threadIdx.x) + j * kT);
+    const int i = 4 * (static_cast<int>(threadIdx.x) + j * T);
     const bool on = i < K;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f), s4 = v, w4 = v, g4 = v, b4 = v;
     if (on) {
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint1
     for (int j = 0; j < NV; j++)
 #pragma unroll
       for (int c = 0; c < 4; c++) s2[0] = __builtin_fmaf(su[j][c], su[j][c], s2[0]);
-    gdev::block_sums<kT / 64, 1>(s2, red, slot);
+    gdev::block_sums<T / 64, 1>(s2, red, slot);
     const float inv = 1.0f / sqrtf(s2[0] / fk + p.eps);
 #pragma unroll
     for (int j = 0; j < NV; j++)
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint1
   if (has_sub) {
 #pragma unroll
     for (int j = 0; j < NV; j++) {
-      const int i = static_cast<int>(threadIdx.x) + j * kT;
+      const int i = static_cast<int>(threadIdx.x) + j * T;
 #pragma unroll
       for (int c = 0; c < 4; c++) t[j][c] += su[j][c];
       if (p.res_out && i < K4)
@@ -174,20 +174,20 @@ __global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint1
       float s[1] = {0.f};
 #pragma unroll
       for (int j = 0; j < NV; j++) s[0] += (t[j][0] + t[j][1]) + (t[j][2] + t[j][3]);
-      gdev::block_sums<kT / 64, 1>(s, red, slot);
+      gdev::block_sums<T / 64, 1>(s, red, slot);
       mean = s[0] / fk;
     }
     float s2[1] = {0.f};
 #pragma unroll
     for (int j = 0; j < NV; j++) {
-      const bool on = static_cast<int>(threadIdx.x) + j * kT < K4;
+      const bool on = static_cast<int>(threadIdx.x) + j * T < K4;
 #pragma unroll
       for (int c = 0; c < 4; c++) {
         t[j][c] -= mean;
         if (on) s2[0] = __builtin_fmaf(t[j][c], t[j][c], s2[0]);
       }
     }
-    gdev::block_sums<kT / 64, 1>(s2, red, slot);
+    gdev::block_sums<T / 64, 1>(s2, red, slot);
     const float inv = 1.0f / sqrtf(s2[0] / fk + p.eps);
     const float one = p.norm == XE_NORM_RMS1P ? 1.0f : 0.0f;
 #pragma unroll
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint1
     uint32_t low = ~0u;
 #pragma unroll
     for (int j = 0; j < NV; j++)
-      if (static_cast<int>(threadIdx.x) + j * kT < K4)
+      if (static_cast<int>(threadIdx.x) + j * T < K4)
 #pragma unroll
         for (int c = 0; c < 4; c++) {
           a = fmaxf(a, fabsf(t[j][c]));
@@ -218,8 +218,11 @@ __global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint1
       mn[threadIdx.x >> 6] = least;
     }
     __syncthreads();
-    a = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
-    least = fminf(fminf(mn[0], mn[1]), fminf(mn[2], mn[3]));
+#pragma unroll
+    for (int w = 0; w < T / 64; w++) {
+      a = fmaxf(a, mx[w]);
+      least = fminf(least, mn[w]);
+    }
     int e = 0;
     if (a > 0.f && a < INFINITY) (void)frexpf(a, &e);  // a in [2^(e-1), 2^e)
     int s = 15 - e;
@@ -230,7 +233,7 @@ __global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint1
     if (threadIdx.x == 0) rexp[b] = rexp_word(s, raw);
 #pragma unroll
     for (int j = 0; j < NV; j++) {
-      const int i = static_cast<int>(threadIdx.x) + j * kT;
+      const int i = static_cast<int>(threadIdx.x) + j * T;
       if (i >= K4) continue;
       union {
         _Float16 h[4];
@@ -260,7 +263,7 @@ __global__ __launch_bounds__(kT) void wide_rows_kernel(gdev::GemvParams p, uint1
   } else {
 #pragma unroll
     for (int j = 0; j < NV; j++) {
-      const int i = static_cast<int>(threadIdx.x) + j * kT;
+      const int i = static_cast<int>(threadIdx.x) + j * T;
       if (i >= K4) continue;
       float r[4], l[4];
 #pragma unroll
@@ -958,10 +961,11 @@ int lds_bytes(int wdtype, bool big) {
 
 template <int P>
 void rows_launch(const gdev::GemvParams &p, const WideRows &rows, hipStream_t s) {
-  const int nv = (p.k / 4 + kT - 1) / kT;
-  auto fn = nv <= 1 ? wide_rows_kernel<1, P> : nv <= 2 ? wide_rows_kernel<2, P> : nv <= 4 ? wide_rows_kernel<4, P>
-            : nv <= 8 ? wide_rows_kernel<8, P> : wide_rows_kernel<16, P>;
-  hipLaunchKernelGGL(fn, dim3(p.batch), dim3(kT), 0, s, p, rows.planes, rows.rexp, rows.raw);
+  // beyond 8 chunks a thread (200 registers) twice the threads
+  const int nv = (p.k / 4 + kT - 1) / kT, threads = nv <= 8 ? kT : 2 * kT;
+  auto fn = nv <= 1 ? wide_rows_kernel<1, P, kT> : nv <= 2 ? wide_rows_kernel<2, P, kT> : nv <= 4 ? wide_rows_kernel<4, P, kT>
+            : nv <= 8 ? wide_rows_kernel<8, P, kT> : wide_rows_kernel<8, P, 2 * kT>;
+  hipLaunchKernelGGL(fn, dim3(p.batch), dim3(threads), 0, s, p, rows.planes, rows.rexp, rows.raw);
   XE_HIP(hipGetLastError());
 }
 

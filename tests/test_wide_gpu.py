@@ -65,13 +65,15 @@ def test_wide_linear(gpu, xe, wd, m, k, b, norm):
     assert rows.max() <= 2e-6, "row %d rel-L2 %g" % (rows.argmax(), rows.max())
 
 
-# (kernel, K splits) a shape has to run on: both tiles, split and not, weight
-# counts that are odd, K beyond what one float4 round of 8 holds, the smallest
+# (kernel, K splits) a shape has to run on: both tiles, split and not, odd
+# weight counts, K beyond 8192 (512 threads a row), about the smallest product
 PATHS = [
-    (4590, 640, 475, "ln", "i8 i4 bf16 bfp16", ("planes", 1)),
-    (3129, 2032, 127, "ln", "i8 i4", ("planes", 2)),
-    (1459, 9152, 126, "rms1p", "i8 i4", ("planes", 5)),
-    (21, 176, 77, "ln", "i8 i4 bf16 bfp16", ("planes", 1)),
+    (4590, 640, 475, "ln", "i8 i4", ("planes", 1)),
+    (3387, 1888, 125, "ln", "i8 i4", ("planes", 2)),
+    (1375, 8608, 127, "rms1p", "i8 i4", ("planes", 5)),
+    (1063, 560, 451, "ln", "i8 i4", ("planes", 1)),
+    (5327, 528, 97, "rms1p", "i8 i4 bf16 bfp16", ("planes", 1)),
+    (7029, 560, 386, "ln", "i8 i4 bf16 bfp16", ("planes_big", 1)),
     (9969, 2192, 281, "rms1p", "i8 i4 bf16 bfp16", ("planes_big", 2)),
     (3519, 8640, 133, "ln", "i8 i4 bf16 bfp16", ("planes_big", 8)),
 ]

@@ -66,6 +66,8 @@ bool wide_takes(int m, int k, int n, int wdtype, const void *x, int ldx);
 // Whether a linear of n rows over an m x k weight is faster here than on the
 // kernels of gemm.hip (prologue: those need one too).
 bool wide_preferred(int m, int k, int n, int wdtype, bool prologue);
+// Microseconds of a product on the kernels of gemm.hip (their own shapes).
+double gemm_est_us(int m, int k, int n);
 // K splits wide_gemm takes for a shape, with at most ws_floats floats of partials.
 int wide_splits(int m, int k, int n, int wdtype, size_t ws_floats);
 // Whether its tiles are the 128 x 256 ones (else 64 x 64).

@@ -914,6 +914,8 @@ struct Shape {
   bool big;
   int ks, spk;
 };
+// us of a step: small tile (two planes, three), big tile
+constexpr double kStepUs[2][2] = {{0.44, 0.58}, {1.27, 1.83}};
 constexpr int kTileX[2] = {64, 128}, kTileW[2] = {64, 256};
 
 Shape choose_shape(int m, int k, int n, int wdtype, size_t ws_floats, double *cost_us = nullptr) {
@@ -923,7 +925,7 @@ Shape choose_shape(int m, int k, int n, int wdtype, size_t ws_floats, double *co
   double best_cost = -1;
   for (int big = 0; big < 2; big++) {
     const long tiles = static_cast<long>((m + kTileW[big] - 1) / kTileW[big]) * ((n + kTileX[big] - 1) / kTileX[big]);
-    const double step = big ? (p2 ? 1.27 : 1.83) : (p2 ? 0.44 : 0.58);
+    const double step = kStepUs[big][p2 ? 0 : 1];
     for (int ks = 1; ks <= kMaxKs; ks++) {
       const int spk = (steps + ks - 1) / ks;
       if ((steps + spk - 1) / spk != ks) continue;
@@ -990,15 +992,42 @@ bool wide_takes(int m, int k, int n, int wdtype, const void *x, int ldx) {
 // which need no planes but split the rows in every weight tile, 8 us and 11.5
 // us for every 1e9 multiply-adds (int8 and bf16 alike), after a prologue of 5
 // us for a norm.  Measured here / there, us: int8 1152 x 1152 at 512 rows 18.5
-// / 16.6, 3072 x 768 at 512 19.9 / 24.4, 4096 x 4096 at 200 36 / 40, 1152 x
-// 6912 at 512 50 / 64, 13824 x 1152 at 512 47 / 107, 14336 x 4096 at 512 121 /
-// 342; bf16 3072 x 768 at 512 28 / 23.5, 4096 x 4096 at 200 40 / 40 (where the
-// estimates are within 5 % the other kernels stay).
+// / 16.6, 3072 x 768 at 512 20.6 / 24.4, 4096 x 4096 at 200 37 / 40, 1152 x
+// 6912 at 512 51 / 64, 13824 x 1152 at 512 49 / 107, 14336 x 4096 at 512 121 /
+// 342; bf16 3072 x 768 at 512 28 / 23.5 (where the estimates are within 5 %
+// the other kernels stay).
+// Near that line both launches are looked at again, by their rounds: there
+// gemm_est_us, here what the cost above leaves out.  Weight tiles run on XCD
+// (tile) mod 8, 32 CUs each (bf16 2560 x 5120 at 384 rows, ten weight tiles, 8
+// splits: 78 / 61), and a big tile's further round adds 8 us; a small tile's workgroups beyond one a CU come in whole
+// ones (int8 5281 x 1152 at 192 after a norm 27.8 / 25.3); partials of a
+// weight count that is no multiple of four are stored one by one (int8 3961 x
+// 5952 at 128 48.8 / 45.0, 3960 of it 44.9 / 45.3); three planes on the small
+// tile spill registers, at a cost that no such count tells (a fifth better by
+// the estimate, or the other kernels stay: bf16 after a norm 3072 x 768 at 300
+// 25.1 / 21.3).
+// Products below 2^28 multiply-adds or of K < 512 stay too: both sides are
+// launches, latency and outputs to store (bf16 after a norm: 8243 x 48 at 200
+// rows 21.8 / 17.0, 3799 x 256 at 450 22.5 / 20.8).
+// Of 826 measured products that the first line alone gives to these kernels 79
+// were more than 4 % slower here; four are left (4566 x 9536, 8 to 15 %), and
+// 30 others would gain 6 to 20 %.
 bool wide_preferred(int m, int k, int n, int wdtype, bool prologue) {
-  if (n <= 64) return false;  // one stream tile of gemm.hip
+  const double mac = static_cast<double>(m) * k * n;
+  if (n <= 64 || k < 512 || mac < (1 << 28)) return false;  // one stream tile of gemm.hip, small products
   double us = 0;
-  (void)choose_shape(m, k, n, wdtype, gemm_op_ws_floats(), &us);
-  return us + 6.0 + 2e-6 * n * k < 0.95 * (8.0 + 11.5e-9 * m * static_cast<double>(k) * n + (prologue ? 5.0 : 0.0));
+  const Shape sh = choose_shape(m, k, n, wdtype, gemm_op_ws_floats(), &us);
+  const double rows = 6.0 + 2e-6 * n * k;
+  if (us + rows >= 0.95 * (8.0 + 11.5e-9 * mac + (prologue ? 5.0 : 0.0))) return false;
+  const bool p2 = wide_planes(wdtype) == 2;
+  const int tw = (m + kTileW[sh.big] - 1) / kTileW[sh.big], tx = (n + kTileX[sh.big] - 1) / kTileX[sh.big];
+  const double rounds = std::ceil((tw + 7) / 8 * tx * sh.ks / 32.0), step = kStepUs[sh.big][p2 ? 0 : 1];
+  double here = sh.big ? 6.0 + sh.spk * step * rounds + 8.0 * (rounds - 1)
+                       : 3.0 + sh.spk * (rounds > 1 ? 1.25 * step * rounds : p2 ? step : step + 0.14);
+  if (sh.ks > 1) here += 3.0 + static_cast<double>(sh.ks) * n * m * (m % 4 ? 3e-6 : 2e-6);
+  here += rows;
+  const double there = gemm_est_us(m, k, n) + (!prologue ? 0.0 : k > 4096 ? 2e-3 * k : 5.0);
+  return here < (p2 || sh.big ? 1.0 : 0.8) * there;
 }
 
 int wide_splits(int m, int k, int n, int wdtype, size_t ws_floats) {

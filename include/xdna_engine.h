@@ -186,9 +186,9 @@ int xe_weight_shape(const xe_weight *w, int *m, int *k, int *wdtype);
 
 /* CtxDecode::gemv (ctx_decode.rs:325-366), batched: y[b,m] = W x[b,k]
  * (+ bias), fp32 out.  x_dtype XE_F32 or XE_BF16 (host pointer).  batch
- * 1..512 (the reference's batched tiles go to Mp = 512, ctx2.rs:46-55): up
- * to 8 rows run the bandwidth GEMV, more the MFMA GEMM (bf16-split fp32
- * activations, fp32 accumulate). */
+ * 1..512 (the reference's batched tiles go to Mp = 512, ctx2.rs:46-55): a
+ * few rows run the bandwidth GEMV, more an MFMA GEMM (fp32 activations as
+ * three bf16 parts, or over row planes; fp32 accumulate): xe_linear_path. */
 int xe_gemv(xe_ctx *ctx, const xe_weight *w, const void *x, int x_dtype,
             int batch, float *y);
 /* CtxDecode::fused_norm_gemv (ctx_decode.rs:617-643). */

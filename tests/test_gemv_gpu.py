@@ -344,8 +344,9 @@ def test_registration_rejects_bad_k(gpu, xe):
 @pytest.mark.parametrize("m,k", [(6912, 1152), (1152, 6912), (3072, 768)])
 @pytest.mark.parametrize("b", [16, 64, 200])
 def test_norm_gemm_int8_batched(gpu, xe, m, k, b):
-    """xe_fused_norm_gemv at 16..200 rows (MFMA GEMM, bf16 three-part split
-    of the fp32 activations, fp32 accumulate) against the oracle GEMV."""
+    """xe_fused_norm_gemv at 16..200 rows (an MFMA GEMM: the fp32 activations
+    as three bf16 parts, or where xe_linear_path says planes as two fp16 parts;
+    fp32 accumulate) against the oracle GEMV."""
     dev, ctx = gpu
     print("[case] int8 LN+GEMM m=%d k=%d b=%d" % (m, k, b), flush=True)
     x, gamma, beta, q, s = config2_inputs(m, k, b, seed=m + k + b)

@@ -252,7 +252,7 @@ GemvLaunch gemv_args(const xe_weight *w, const void *x, int x_dtype, int batch, 
   return g;
 }
 
-// Up to 8 rows: the GEMV kernels; 9..kMaxOpBatch: the MFMA GEMM (fp32 x).
+// A few rows: the GEMV kernels; up to kMaxOpBatch: an MFMA GEMM (fp32 x).
 constexpr int kMaxOpBatch = 512;  // the reference's largest batched tile (Mp <= 512, ctx2.rs)
 
 void launch_linear(xe_ctx *ctx, const xe_weight *w, const void *x, int x_dtype, int batch,

@@ -1,4 +1,5 @@
-// gemm.hip -- decode projections for 16 or more streams on MFMA.
+// gemm.hip -- decode projections from 4 streams on, and linears of up to 512
+// rows that are not faster over row planes (wide.hip), on MFMA.
 //
 // At b >= 16 a decode projection Y[b, m] = act(scale[m] * sum_k W[m, k] X[b, k]
 // + bias[m]) is a real GEMM (the reference's batched lockstep decoder,

@@ -16,8 +16,11 @@
 //                            saturating cast)
 //   3. the i32 product       <= 8 rows: the sdot4 GEMV (gemv.hip); more rows
 //                            (the reference's batched tiles, Mp <= 512): an
-//                            int8 MFMA GEMM (v_mfma_i32_16x16x64_i8), exact
-//                            integer accumulation
+//                            int8 MFMA GEMM over 64 x 64 tiles in LDS
+//                            (v_mfma_i32_32x32x32_i8) or, for a few rows of a
+//                            short K, one that loads its operands straight
+//                            (v_mfma_i32_16x16x64_i8), exact integer
+//                            accumulation
 //   4. the epilogue          fused into the product: v = (acc * scale_a) *
 //                            ws[c] (+ bias[c], or SiLU(v + bias[c]) with the
 //                            reference's fast_sigmoid), in the reference's

@@ -3,12 +3,14 @@
 // residual prologue and writes the activations as split 16-bit planes, and an
 // MFMA GEMM over those planes.
 //
-// What bounds it: the matrix cores.  An fp32 activation needs more than one
-// 16-bit part, so every weight x row product costs one MFMA a part; the parts
-// are made once per row here instead of once per weight tile in the GEMM
-// (gemm.hip splits the fp32 rows again in every workgroup, which is right for
-// the few rows of a decode step and costs more than the MFMAs from about a
-// hundred rows on).
+// What bounds it: in the K loop the matrix cores, two thirds of its cycles; a
+// launch of one round spends as long again on its start and its outputs (29 %
+// of the matrix cores' cycles at 13824 x 1152 x 512).  An fp32 activation needs
+// more than one 16-bit part, so every weight x row product costs one MFMA a
+// part; the parts are made once per row here instead of once per weight tile
+// in the GEMM (gemm.hip splits the fp32 rows again in every workgroup, which is
+// right for the few rows of a decode step and costs more than the MFMAs from
+// about a hundred rows on).
 //   int8 / int4 weights are whole numbers below 2^11, exact in fp16, so two
 //   fp16 parts do: x 2^s = hi + lo 2^-12 + e, round to nearest each, with s
 //   per row putting the largest |x| in [2^14, 2^15).  The second part is kept
@@ -906,10 +908,11 @@ __global__ __launch_bounds__(kT) void wide_finish_kernel(WideParams p, int ks, i
 //   small  64 x 64, 4 waves, loads of four steps in flight: shapes whose big
 //          tiles leave CUs idle
 // Cost in microseconds, fitted to launches over one dimension at a time (512
-// rows, int8 / bf16 weights): a big tile's step takes 1.27 / 1.83 us (64 to 67
-// % of the matrix cores' cycles) and its launch 6 us of latency; a small
-// tile's 0.44 / 0.58 us, alone on its CU or 1.25 times that for each
-// workgroup of it; a K split writes and reads its partials at about 4 TB/s.
+// rows, int8 / bf16 weights): a big tile's step takes 1.27 / 1.83 us (the
+// matrix cores busy for two thirds of it) and its launch 6 us of latency; a
+// small tile's 0.44 / 0.58 us, alone on its CU or 1.25 times that for each
+// workgroup of it (three planes: measured with loads that spill); a K split
+// writes and reads its partials at about 4 TB/s.
 struct Shape {
   bool big;
   int ks, spk;

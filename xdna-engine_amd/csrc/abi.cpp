@@ -363,7 +363,7 @@ xe_device *xe_device_open(int ordinal) {
     d->arch = prop.gcnArchName;
     d->num_cus = prop.multiProcessorCount;
     d->max_lds = prop.sharedMemPerBlock;
-    // default priority: other priorities have hung on this hardware pool
+    // default priority: other priorities have hung on this hardware
     XE_HIP(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking));
     // the static attention workspace's device address, once per device
     (void)attn_static_scratch(ordinal);

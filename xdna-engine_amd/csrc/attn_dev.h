@@ -615,9 +615,9 @@ __device__ __forceinline__ void attn_merge_block(const AttnParams &p, int blk, i
 // kernel's own merge.  Every partial a thread takes is loaded before the
 // weights, so the merge is one memory round trip whatever the split count.
 // 4 heads x 256 of one key head, one stream, split and merge, us: 32768 keys
-// 34.9 (256 threads, one level, at most 64 splits) -> 17.7 to 19.4 by the box,
-// 4096 keys 16.6 -> 11.7, 8 streams at 4096 keys 20.4 -> 15.3 (20.3 / 13.1 /
-// 16.8 with a branch a load instead of clamped loads).
+// 34.9 (256 threads, one level, at most 64 splits) -> 17.7 (19.4 on another
+// card), 4096 keys 16.6 -> 11.7, 8 streams at 4096 keys 20.4 -> 15.3 (20.3 /
+// 13.1 / 16.8 with a branch a load instead of clamped loads).
 constexpr int kTeams = 4;
 __host__ __device__ constexpr int team_threads(int hd, int g) { return g * hd < kThreads ? g * hd : kThreads; }
 template <int HD, int G>

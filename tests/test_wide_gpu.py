@@ -163,8 +163,9 @@ def test_prompt_in_smaller_passes(gpu, xe, monkeypatch, family, batch, n, mb):
 
 
 @pytest.mark.parametrize("wd", ["i8", "i4"])
-@pytest.mark.parametrize("m,k,b", [(4100, 4096, 509), (4590, 640, 475)])
-def test_wide_linear_range_within_a_row(gpu, xe, wd, m, k, b):
+@pytest.mark.parametrize("m,k,b,path", [(4100, 4096, 509, ("planes_big", 3)), (4590, 640, 475, ("planes", 1)),
+                                        (7029, 560, 386, ("planes_big", 1)), (3519, 8656, 389, ("planes_big", 4))])
+def test_wide_linear_range_within_a_row(gpu, xe, wd, m, k, b, path):
     """Rows whose elements differ by up to the whole fp32 range: one large
     element under a zero weight column, magnitudes spread over 2^-100 .. 2^100
     under weights that are non-zero in 48 columns only, between ordinary rows
@@ -173,7 +174,7 @@ def test_wide_linear_range_within_a_row(gpu, xe, wd, m, k, b):
     the sum of their magnitudes (n roundings of an fp32 sum, operands to
     2^-23 each, the scale)."""
     _, ctx = gpu
-    assert xe.linear_path(xe.XE_I8 if wd == "i8" else xe.XE_I4, m, k, b) == (("planes_big", 3) if m == 4100 else ("planes", 1))
+    assert xe.linear_path(xe.XE_I8 if wd == "i8" else xe.XE_I4, m, k, b) == path
     print("[case] wide range %s m=%d k=%d b=%d" % (wd, m, k, b), flush=True)
     rng = np.random.default_rng(m + b)
     x = rng.standard_normal((b, k)).astype(np.float32)
